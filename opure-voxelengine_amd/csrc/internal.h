@@ -16,7 +16,11 @@
 //  Host side: device object, errors, workspace
 // ---------------------------------------------------------------------------
 constexpr uint32_t REJ_SYNC_SEQS = 4096;
-constexpr uint64_t REJ_SYNC_BYTES = REJ_SYNC_SEQS * 4ull + REJ_SYNC_SEQS * 64ull * 6ull * 8ull;
+// the sliced sampler's state: a launch count a row, then [SMP_SYNC_ROWS][64
+// slices][3] tagged words; at the end of the rejection sampler's
+constexpr uint32_t SMP_SYNC_ROWS = 4096;
+constexpr uint64_t SMP_SYNC_BYTES = SMP_SYNC_ROWS * 4ull + SMP_SYNC_ROWS * 64ull * 3ull * 8ull;
+constexpr uint64_t REJ_SYNC_BYTES = REJ_SYNC_SEQS * 4ull + REJ_SYNC_SEQS * 64ull * 6ull * 8ull + SMP_SYNC_BYTES;
 // The LM head's in-launch greedy acceptance: tagged (value, index) words of
 // up to ACC_SYNC_WGS workgroups x OPURE_MAX_ROWS rows, then the launch count
 constexpr uint32_t ACC_SYNC_WGS = 4096;
@@ -40,7 +44,9 @@ struct opure_dev {
     // The one-launch rejection sampler's per-sequence state (REJ_SYNC_BYTES,
     // zeroed once at creation): a launch count a sequence [REJ_SYNC_SEQS] u32,
     // then the sequences' slots [REJ_SYNC_SEQS][64 slices][6] u64, whose tags
-    // carry the launch count, so no clear is needed between launches.
+    // carry the launch count, so no clear is needed between launches; then
+    // the sliced sampler's (SMP_SYNC_BYTES).  Zeroed again after a bounded
+    // wait gave up (check_device_errors).
     void*       rej_sync = nullptr;
     // The LM head's in-launch greedy acceptance state (ACC_SYNC_BYTES): the
     // workgroups' tagged words, zeroed, then the launch count, which starts

@@ -81,9 +81,10 @@ int check_device_errors(opure_dev* dev)
     for (uint32_t i = 0; i < ERR_WORDS; ++i) { w[i] = dev->err[i]; dev->err[i] = 0u; }
     if (w[ERR_WAIT] && dev->acc_sync && !dev->capturing)
     {
-        // a given-up in-launch acceptance may leave words a later launch would
-        // take for its own: start that state afresh (the stream is idle here)
+        // a launch that gave up may leave words a later launch would take for
+        // its own: start the exchanged state afresh (the stream is idle here)
         hipError_t e = reset_acc_sync(dev);
+        if (e == hipSuccess && dev->rej_sync) e = hipMemsetAsync(dev->rej_sync, 0, REJ_SYNC_BYTES, dev->stream);
         if (e == hipSuccess) e = hipStreamSynchronize(dev->stream);
         if (e != hipSuccess) return hip_fail(e, "resetting the in-launch acceptance state");
     }

@@ -868,6 +868,41 @@ def test_sample_rows_and_philox_bit_exact(dev):
     assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("rows,V,tau,off", [
+    (3, 1, 0.7, 0), (2, 3, 1.0, 1), (5, 4095, 0.8, 0), (5, 4096, 0.8, 0), (5, 4097, 1.0, 0), (3, 8192, 0.5, 1),
+    (4, 128256, 0.8, 0), (1, 128263, 1.0, 0), (2, 262144, 0.9, 0), (2, 262145, 0.9, 0), (5000, 64, 0.8, 0)],
+    ids=lambda v: str(v))
+def test_sample_rows_slices_bit_exact(dev, rows, V, tau, off):
+    """Rows of one slice, whole slices, a remainder, the most slices and one
+    past them (one workgroup a row), logits off 16-byte alignment, more rows
+    than one launch takes; rows of no mass (all -inf, NaN, an infinity) and a
+    row whose mass is in its last id.  Ids equal the oracle's, and again on the
+    next launch (whose words carry another count)."""
+    say("sample slices", rows, V, tau, off)
+    rng = np.random.default_rng(V + rows)
+    lg = (rng.standard_normal((rows, V)) * 2).astype(np.float32)
+    if rows > 1:
+        lg[1] = -np.inf
+        lg[1, -1] = 3.0
+    if rows > 2:
+        lg[2] = -np.inf
+    if rows > 3:
+        lg[3, 0] = np.nan
+        lg[3, V // 2] = np.nan
+    if rows > 4:
+        lg[4, V // 3] = np.inf
+    pos = rng.integers(0, 1 << 20, rows).astype(np.uint32)
+    seq = rng.integers(0, 64, rows).astype(np.uint32)
+    buf = dev.upload(np.concatenate([np.zeros(off, np.float32), lg.ravel()]))
+    pb, sb, ob = dev.upload(pos), dev.upload(seq), dev.alloc(rows * 4)
+    want = O.sample_rows(lg, tau, 12, pos, seq, 1)
+    a = H.SampleArgs(rows, V, int(buf) + 4 * off, tau, 12, int(pb), int(sb), 1, int(ob))
+    for _ in range(2):
+        H.check(H.lib().opure_sample_rows(dev.h, C.byref(a)))
+        dev.sync()
+        assert np.array_equal(dev.download(ob, np.int32, (rows,)), want)
+
+
 def test_rollback_bit_exact(dev):
     hm = O.HostModel(n_layers=2, hidden=64, n_heads=4, n_kv_heads=2, head_dim=32, ffn=64, vocab=64,
                      wfmt=O.W_I8PC, afmt=O.A_F16, seed=3)
