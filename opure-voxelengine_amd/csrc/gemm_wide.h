@@ -9,10 +9,10 @@
 //  Work split.  A workgroup owns 8 consecutive 16-row weight tiles (a row
 //  group), up to 8 16-column tiles of X (a column group) and one range of K
 //  blocks (a split; shapes with few row groups split K so the CUs fill).  A
-//  set of 4 waves covers the row group: wave w multiplies tiles 2w, 2w + 1 by
-//  all of the group's column tiles, so it keeps 16 accumulator tiles, loads
-//  each weight byte once and reads each B fragment once per block for two
-//  MFMAs.  Weights go straight from HBM into registers: every wave loads its
+//  set of 4 waves covers the row group (more than 64 rows of X): wave w multiplies
+//  tiles 2w, 2w + 1 by all of the group's column tiles, so it keeps 16 accumulator
+//  tiles, loads each weight byte once and reads each B fragment once per block for
+//  two MFMAs.  Fewer rows take one weight tile a wave (WideShape).  Weights go straight from HBM into registers: every wave loads its
 //  own two tiles' 16 bytes a lane per block, in static register slots DW
 //  blocks ahead.  X goes through LDS: per block the set loads its column
 //  group's fragments into registers DX blocks ahead and writes them into a
@@ -41,30 +41,45 @@
 
 namespace opure_gemv {
 
-constexpr uint32_t WIDE_WR = 4, WIDE_WC = 1;     // wave grid of a K half: wave rows x wave columns
-constexpr uint32_t WIDE_TA = 2;                  // weight tiles per wave
-constexpr uint32_t WIDE_TB = 8;                  // column tiles per wave
-constexpr uint32_t WIDE_RT = WIDE_WR * WIDE_TA;  // weight tiles per workgroup
-constexpr uint32_t WIDE_CG = WIDE_WC * WIDE_TB;  // column tiles per workgroup at most
+constexpr uint32_t WIDE_RT = 8;       // weight tiles of the plan's row groups (the K splits follow from these)
+constexpr uint32_t WIDE_CG = 8;       // column tiles per workgroup at most
 constexpr uint32_t WIDE_MAX_M = 256;  // rows of X
+
+// The wave grid: a set of 4 waves is 4 / WC wave rows x WC wave columns, each
+// wave TA weight tiles x TB column tiles.  CT = WC * TB column tiles a
+// workgroup; RT = (4 / WC) * TA weight tiles.
+//   CT 8: the general shape (128 x 128 outputs a workgroup)
+//   CT 4, 2: a batch of at most 64 / 32 rows, which is bound by the weight
+//     stream: no matrix work on column tiles that are not there, and at one
+//     tile a wave twice the workgroups (8B o_proj, 4 splits: 128 -> 256), so
+//     every CU loads: uint4 gate/up 28,672 x 4,096 at 24 rows 77.5 -> 26.3 us.
+template <uint32_t TA_, uint32_t TB_, uint32_t WC_> struct WideShape {
+    static constexpr uint32_t TA = TA_, TB = TB_, WC = WC_, RT = (4u / WC_) * TA_, CT = WC_ * TB_;
+};
 
 // register slots of the software pipeline: DW weight blocks and DX X blocks
 // in flight; the K loop is unrolled by U = lcm(DW, DX), an even number, so
 // slots and LDS stages are compile-time.  KH = 2 runs two sets of 4 waves on
 // alternate K blocks (two waves a SIMD: one issues MFMAs while the other
-// waits); the uint4 kernel's registers leave room for one.
-template <int WF> struct WideDepth;
-template <> struct WideDepth<OPURE_W_I8PC>   { static constexpr uint32_t DW = 4, DX = 2, U = 4, KH = 2; };
-template <> struct WideDepth<OPURE_W_I4G128> { static constexpr uint32_t DW = 2, DX = 1, U = 2, KH = 1; };
+// waits); the uint4 kernel's registers leave room for one.  PU: the plan's
+// splits are multiples of PU blocks.
+template <int WF, uint32_t CT> struct WideDepth;
+template <uint32_t CT> struct WideDepth<OPURE_W_I8PC, CT>   { static constexpr uint32_t DW = 4, DX = 2, U = 4, KH = 2, PU = 4; };
+template <uint32_t CT> struct WideDepth<OPURE_W_I4G128, CT>
+{
+    static constexpr uint32_t DW = CT == 8u ? 2 : 4, DX = CT == 8u ? 1 : 2, U = CT == 8u ? 2 : 4, KH = 1, PU = 2;
+};
+
+constexpr uint32_t wide_threads(int wf) { return wf == OPURE_W_I8PC ? 512u : 256u; }   // 256 KH
 
 struct WParams {
     KParams p;        // shape, pointers, epilogue
     uint32_t mt;      // 16-column tiles of X
-    uint32_t nrg;     // row groups (WIDE_RT tiles each)
+    uint32_t nrg;     // row groups (the kernel shape's RT tiles each)
     uint32_t ncg;     // column groups
     uint32_t cgs;     // column tiles per group (<= WIDE_CG)
     uint32_t splits;  // K splits
-    uint32_t bps;     // blocks per split, a multiple of WideDepth::U
+    uint32_t bps;     // blocks per split
     uint32_t part_rows;  // splits > 1: 0 = accumulators [split][tile][mt][64] lanes, 1 = [split][M][out] rows
     f4_t* part;       // splits > 1: the splits' accumulators
 };
@@ -84,33 +99,35 @@ __device__ __forceinline__ void wide_coords(const WParams& wp, uint32_t& split, 
     split = rest / wp.nrg;
 }
 
-template <int WF, int AF, int EPI>
-__global__ __launch_bounds__(256 * WideDepth<WF>::KH) void k_gemm_wide(WParams wp)
+template <int WF, int AF, int EPI, class SH>
+__global__ __launch_bounds__(wide_threads(WF)) __attribute__((amdgpu_waves_per_eu(2))) void k_gemm_wide(WParams wp)
 {
     static_assert(WF == OPURE_W_I8PC || WF == OPURE_W_I4G128, "the wide GEMV reads quantised weights");
     constexpr uint32_t KB = Fmt<WF>::KB;
     constexpr uint32_t NMF = KB / 32u;             // MFMAs (16-byte B fragments) per block per tile pair
     constexpr uint32_t CH = KB / 8u;               // 16-byte X chunks per row per block
-    constexpr uint32_t XR = WIDE_CG * 16u * CH / 256u;  // X chunks a thread stages per block
-    constexpr uint32_t STAGE = WIDE_CG * NMF * 64u;     // u4_t per LDS stage
-    constexpr uint32_t DW = WideDepth<WF>::DW, DX = WideDepth<WF>::DX, U = WideDepth<WF>::U;
-    constexpr uint32_t KH = WideDepth<WF>::KH;
-    constexpr uint32_t TA = WIDE_TA, TB = WIDE_TB;
-    static_assert(WIDE_WR * WIDE_WC == 4 && TA % 2 == 0, "a K half is 4 waves");
-    static_assert(KH == 1 || 2u * STAGE * 2u >= 2u * 4u * (TA / 2u) * TB * 64u, "the halves' exchange reuses the X stages");
+    constexpr uint32_t TA = SH::TA, TB = SH::TB, WC = SH::WC, RT = SH::RT, CT = SH::CT;
+    constexpr uint32_t XR = CT * 16u * CH / 256u;  // X chunks a thread stages per block
+    constexpr uint32_t STAGE = CT * NMF * 64u;     // u4_t per LDS stage
+    using WD = WideDepth<WF, CT>;
+    constexpr uint32_t DW = WD::DW, DX = WD::DX, U = WD::U, KH = WD::KH;
+    constexpr bool GS = WF == OPURE_W_I4G128;      // group sums of X
+    static_assert(XR >= 1 && TB % 2 == 0, "whole chunks a thread; the halves exchange half of the column tiles");
+    static_assert(KH == 1 || 4u * TA * TB * 64u <= KH * 2u * STAGE, "the halves' exchange reuses the X stages");
+    static_assert(!GS || CH == 16u, "a DPP row of lanes stages one X row's group");
     __shared__ u4_t xl[KH * 2 * STAGE];
+    __shared__ float xsl[GS ? 2 : 1][GS ? CT * 16u : 1u];   // uint4: each stage's group sums of X
     const KParams& p = wp.p;
     const uint32_t tid = threadIdx.x & 255u, lane = tid & 63u, g4 = lane >> 4, r16 = lane & 15u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t kh = wave >> 2, w4 = wave & 3u;            // K half, wave within the half
-    const uint32_t wr = w4 / WIDE_WC, wc = w4 % WIDE_WC;
+    const uint32_t wr = w4 / WC, wc = w4 % WC;
     const uint32_t nblk = p.nblk, G = p.in / 128u;
     uint32_t split, rg, cg;
     wide_coords(wp, split, rg, cg);
     const uint32_t ct0 = cg * wp.cgs;
-    const uint32_t cn = min(wp.cgs, wp.mt - ct0);            // column tiles of this group
-    const uint32_t tb = cn > wc ? (cn - wc + WIDE_WC - 1u) / WIDE_WC : 0u;  // of this wave: local wc, wc + WC, ...
-    const uint32_t tile0 = rg * WIDE_RT + wr * TA;
+    const uint32_t cn = min(wp.cgs, wp.mt - ct0);            // column tiles of this group; of this wave: TB wc + j
+    const uint32_t tile0 = rg * RT + wr * TA;
     const uint32_t b_begin = split * wp.bps, b_end = min(nblk, b_begin + wp.bps);
     u4_t* xh = xl + kh * 2u * STAGE;                          // this half's two stages
 
@@ -118,16 +135,16 @@ __global__ __launch_bounds__(256 * WideDepth<WF>::KH) void k_gemm_wide(WParams w
     // wave's load covers 8 rows x 128 contiguous bytes).  In LDS, chunk c of row rr sits at row
     // slot rr ^ c of its fragment: the 8 chunks of a row land in 8 bank groups, and a fragment
     // read (lane (g4, r16) takes chunk NMF g4 + q of row r16) still reads 16 distinct slots.
+    // Rows past M (or past the group's column tiles) read row M - 1 again: their columns are
+    // computed and never stored.
     uint64_t xrow[XR];
     uint32_t xdst[XR];
-    bool xzero[XR];
 #pragma unroll
     for (uint32_t u = 0; u < XR; ++u)
     {
         const uint32_t e = u * 256u + tid;
         const uint32_t c = e % CH, rr = (e / CH) & 15u, ctl = e / (16u * CH);
         const uint32_t m = 16u * (ct0 + ctl) + rr;
-        xzero[u] = ctl >= cn || m >= p.M;
         xrow[u] = (static_cast<uint64_t>(min(m, p.M - 1u)) * p.in + 8u * c) * 2u;
         xdst[u] = (ctl * NMF + c % NMF) * 64u + (c / NMF) * 16u + (rr ^ (c & 15u));
     }
@@ -136,9 +153,35 @@ __global__ __launch_bounds__(256 * WideDepth<WF>::KH) void k_gemm_wide(WParams w
 #pragma unroll
         for (uint32_t u = 0; u < XR; ++u) v[u] = *reinterpret_cast<const u4_t*>(p.x + xrow[u] + k0);
     };
+    // uint4: the group's sum of X of a row, once a workgroup here instead of
+    // in every wave beside its MFMAs (it was 38% of the loop's vector
+    // instructions, which bound the loop; uint4 gate/up 28,672 x 4,096 at 256
+    // rows 165 -> 95 us with the fresh group accumulators kept to one column
+    // tile and out of the accumulation registers).  The 16 lanes of a DPP row stage one row: chunk c = 4 g +
+    // q is MFMA q's share of lane group g; the sums over q in order, then
+    // (g0 + g1) + (g2 + g3).
     auto xstore = [&](const u4_t (&v)[XR], uint32_t st) {
+        float t[XR];
 #pragma unroll
-        for (uint32_t u = 0; u < XR; ++u) xh[st * STAGE + xdst[u]] = xzero[u] ? u4_t{0u, 0u, 0u, 0u} : v[u];
+        for (uint32_t u = 0; u < XR; ++u)
+        {
+            xh[st * STAGE + xdst[u]] = v[u];
+            if constexpr (GS)
+            {
+                const float s = unit_sum<AF>(v[u][0], v[u][1], v[u][2], v[u][3]);
+                t[u] = dpp_f<0x00>(s) + dpp_f<0x55>(s);
+                t[u] += dpp_f<0xAA>(s);
+                t[u] += dpp_f<0xFF>(s);
+                t[u] += dpp_f<0x141>(t[u]);   // row_half_mirror: g ^ 1
+                t[u] += dpp_f<0x140>(t[u]);   // row_mirror: the other pair
+            }
+        }
+        if constexpr (GS)
+        {
+            if ((tid & 15u) == 0u)
+#pragma unroll
+                for (uint32_t u = 0; u < XR; ++u) xsl[st][u * 16u + (tid >> 4)] = t[u];
+        }
     };
 
     // this wave's weight tiles (clamped for loads; the epilogue skips tiles past the end)
@@ -167,98 +210,100 @@ __global__ __launch_bounds__(256 * WideDepth<WF>::KH) void k_gemm_wide(WParams w
 #pragma unroll
         for (uint32_t j = 0; j < TB; ++j) acc[a][j] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
-    // one block: B fragments from LDS stage st, A decoded from the weight registers
+    auto mma = [&](const u4_t& a, const u4_t& b, const f4_t& c) -> f4_t {
+        if constexpr (AF == OPURE_A_F16)
+            return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a), __builtin_bit_cast(half8_t, b), c, 0, 0, 0);
+        else
+            return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+    };
+    // one block: B fragments from LDS stage st, A decoded from the weight
+    // registers.  Every wave runs all TB column slots (a slot past the group
+    // is never stored): no branches between MFMAs.
     auto compute = [&](const u4_t (&w)[TA], const u4_t (&s)[TA], uint32_t st) {
         const u4_t* xb = xh + st * STAGE;
-        f4_t bacc[TA][TB];
-        float xpart[TB];
-        if constexpr (WF == OPURE_W_I4G128)
+        auto frag = [&](uint32_t j, uint32_t q) {
+            return xb[((TB * wc + j) * NMF + q) * 64u + g4 * 16u + (r16 ^ ((NMF * g4 + q) & 15u))];
+        };
+        if constexpr (!GS)
         {
 #pragma unroll
-            for (uint32_t a = 0; a < TA; ++a)
-#pragma unroll
-                for (uint32_t j = 0; j < TB; ++j) bacc[a][j] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (uint32_t j = 0; j < TB; ++j) xpart[j] = 0.0f;
-        }
-#pragma unroll
-        for (uint32_t q = 0; q < NMF; ++q)
-        {
-            u4_t bf[TB];
-#pragma unroll
-            for (uint32_t j = 0; j < TB; ++j)
-                bf[j] = xb[(min(wc + WIDE_WC * j, WIDE_CG - 1u) * NMF + q) * 64u + g4 * 16u + (r16 ^ ((NMF * g4 + q) & 15u))];
-            if constexpr (WF == OPURE_W_I4G128)
+            for (uint32_t q = 0; q < NMF; ++q)
             {
+                u4_t bf[TB];
 #pragma unroll
-                for (uint32_t j = 0; j < TB; ++j) xpart[j] += unit_sum<AF>(bf[j][0], bf[j][1], bf[j][2], bf[j][3]);
-            }
+                for (uint32_t j = 0; j < TB; ++j) bf[j] = frag(j, q);
 #pragma unroll
-            for (uint32_t a = 0; a < TA; ++a)
-            {
-                u4_t af;
-                if constexpr (WF == OPURE_W_I8PC)
+                for (uint32_t a = 0; a < TA; ++a)
                 {
                     uint32_t o[4];
                     u8x4_to_f16(w[a][2u * q], o[0], o[1]);
                     u8x4_to_f16(w[a][2u * q + 1u], o[2], o[3]);
-                    af = u4_t{o[0], o[1], o[2], o[3]};
-                }
-                else
-                {
-                    uint32_t o[4];
-                    u4x8_pairs<AF>(w[a][q], o);
-                    af = u4_t{o[0], o[1], o[2], o[3]};
-                }
-                // every wave runs all TB column slots (a slot past the group reads a
-                // clamped fragment and is never stored): no branches between MFMAs
+                    const u4_t af = {o[0], o[1], o[2], o[3]};
 #pragma unroll
-                for (uint32_t j = 0; j < TB; ++j)
-                {
-                    if constexpr (WF == OPURE_W_I8PC)
-                        acc[a][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, af),
-                                                                           __builtin_bit_cast(half8_t, bf[j]), acc[a][j], 0, 0, 0);
-                    else if constexpr (AF == OPURE_A_F16)
-                        bacc[a][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, af),
-                                                                            __builtin_bit_cast(half8_t, bf[j]), bacc[a][j], 0, 0, 0);
-                    else
-                        bacc[a][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, af),
-                                                                             __builtin_bit_cast(bf16x8_t, bf[j]), bacc[a][j], 0, 0, 0);
+                    for (uint32_t j = 0; j < TB; ++j) acc[a][j] = mma(af, bf[j], acc[a][j]);
                 }
             }
         }
-        if constexpr (WF == OPURE_W_I4G128)
+        else
         {
-            // acc += (s / MUL) * (bacc - (OFF + MUL z) * xs), xs = the block's sum of X for this column (see U4)
+            // a column tile at a time, so that the fresh group accumulators
+            // take 4 TA registers instead of 4 TA TB
+            u4_t af[TA][NMF];
+            f4_t sc[TA], zo[TA];
+#pragma unroll
+            for (uint32_t a = 0; a < TA; ++a)
+            {
+#pragma unroll
+                for (uint32_t q = 0; q < NMF; ++q)
+                {
+                    uint32_t o[4];
+                    u4x8_pairs<AF>(w[a][q], o);
+                    af[a][q] = u4_t{o[0], o[1], o[2], o[3]};
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                {
+                    float c, z;
+                    u4_group<AF>(s[a][i], c, z);
+                    sc[a][i] = c;
+                    zo[a][i] = z;
+                }
+            }
 #pragma unroll
             for (uint32_t j = 0; j < TB; ++j)
             {
-                const float xs = add_xor32(add_xor16(xpart[j]));
+                u4_t bf[NMF];
+#pragma unroll
+                for (uint32_t q = 0; q < NMF; ++q) bf[q] = frag(j, q);
+                const float xs = xsl[st][16u * (TB * wc + j) + r16];
+                f4_t bacc[TA];
+#pragma unroll
+                for (uint32_t a = 0; a < TA; ++a) bacc[a] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (uint32_t q = 0; q < NMF; ++q)
+#pragma unroll
+                    for (uint32_t a = 0; a < TA; ++a) bacc[a] = mma(af[a][q], bf[q], bacc[a]);
+                // acc += (s / MUL) * (bacc - (OFF + MUL z) * xs), xs = the block's sum of X for this column (see U4)
 #pragma unroll
                 for (uint32_t a = 0; a < TA; ++a)
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
-                    {
-                        float sc, zo;
-                        u4_group<AF>(s[a][i], sc, zo);
-                        acc[a][j][i] = __fmaf_rn(sc, __fmaf_rn(-zo, xs, bacc[a][j][i]), acc[a][j][i]);
-                    }
+                        acc[a][j][i] = __fmaf_rn(sc[a][i], __fmaf_rn(-zo[a][i], xs, bacc[a][i]), acc[a][j][i]);
             }
         }
     };
 
     // int8 with one split: the row scales of the tiles this wave finishes, loaded
     // now rather than after the K loop (a round trip off the epilogue)
-    constexpr uint32_t FT = KH == 1 ? TA : TA / 2u;      // tiles a wave finishes
-    f4_t scl[FT];
+    f4_t scl[TA];
     if constexpr (WF == OPURE_W_I8PC)
     {
 #pragma unroll
-        for (uint32_t h = 0; h < FT; ++h)
+        for (uint32_t a = 0; a < TA; ++a)
         {
-            const uint32_t t = min(tile0 + (KH == 1 ? h : kh * FT + h), p.tiles - 1u);
+            const uint32_t t = min(tile0 + a, p.tiles - 1u);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) scl[h][i] = f16_to_f32(static_cast<const uint16_t*>(p.sc)[t * 16u + 4u * g4 + i]);
+            for (int i = 0; i < 4; ++i) scl[a][i] = f16_to_f32(static_cast<const uint16_t*>(p.sc)[t * 16u + 4u * g4 + i]);
         }
     }
 
@@ -286,16 +331,15 @@ __global__ __launch_bounds__(256 * WideDepth<WF>::KH) void k_gemm_wide(WParams w
         }
     }
 
-    // a: the tile within the wave's TA, h: its index among the FT it finishes
-    auto finish = [&](uint32_t a, uint32_t h, uint32_t j, const f4_t& tot) {
-        const uint32_t tile = tile0 + a;
-        if (tile >= p.tiles || j >= tb) return;
-        const uint32_t ct = ct0 + wc + WIDE_WC * j;
+    auto finish = [&](uint32_t a, uint32_t j, const f4_t& tot) {
+        const uint32_t tile = tile0 + a, cl = TB * wc + j;
+        if (tile >= p.tiles || cl >= cn) return;
+        const uint32_t ct = ct0 + cl;
         if (wp.splits == 1u)
         {
             float bv = 0.0f;
             int32_t bi = 0;
-            epilogue<WF, EPI>(p, tile, 16u * ct + r16, g4, tot, bv, bi, WF == OPURE_W_I8PC ? &scl[h] : nullptr);
+            epilogue<WF, EPI>(p, tile, 16u * ct + r16, g4, tot, bv, bi, WF == OPURE_W_I8PC ? &scl[a] : nullptr);
         }
         else if (wp.part_rows)
         {
@@ -314,33 +358,33 @@ __global__ __launch_bounds__(256 * WideDepth<WF>::KH) void k_gemm_wide(WParams w
 #pragma unroll
         for (uint32_t a = 0; a < TA; ++a)
 #pragma unroll
-            for (uint32_t j = 0; j < TB; ++j) finish(a, a, j, acc[a][j]);
+            for (uint32_t j = 0; j < TB; ++j) finish(a, j, acc[a][j]);
     }
     else
     {
         // the halves add through LDS (the X stages are free): half 0 finishes
-        // the first TA/2 tiles of its wave, half 1 the others; each sum is
-        // (even blocks) + (odd blocks)
-        constexpr uint32_t HT = TA / 2u;
+        // the first TB/2 column tiles of its wave, half 1 the others; each sum
+        // is (even blocks) + (odd blocks)
+        constexpr uint32_t HB = TB / 2u;
         __syncthreads();
-        u4_t* ex = xl + ((1u - kh) * 4u + w4) * (HT * TB * 64u);  // the other half's inbox for this wave
+        u4_t* ex = xl + ((1u - kh) * 4u + w4) * (TA * HB * 64u);  // the other half's inbox for this wave
 #pragma unroll
-        for (uint32_t h = 0; h < HT; ++h)
+        for (uint32_t a = 0; a < TA; ++a)
 #pragma unroll
-            for (uint32_t j = 0; j < TB; ++j)
-                ex[(h * TB + j) * 64u + lane] = __builtin_bit_cast(u4_t, kh == 0 ? acc[HT + h][j] : acc[h][j]);
+            for (uint32_t j = 0; j < HB; ++j)
+                ex[(a * HB + j) * 64u + lane] = __builtin_bit_cast(u4_t, kh == 0 ? acc[a][HB + j] : acc[a][j]);
         __syncthreads();
-        const u4_t* in = xl + (kh * 4u + w4) * (HT * TB * 64u);
-        const uint32_t keep = kh == 0 ? 0u : HT;
+        const u4_t* in = xl + (kh * 4u + w4) * (TA * HB * 64u);
+        const uint32_t keep = kh == 0 ? 0u : HB;
 #pragma unroll
-        for (uint32_t h = 0; h < HT; ++h)
+        for (uint32_t a = 0; a < TA; ++a)
 #pragma unroll
-            for (uint32_t j = 0; j < TB; ++j)
+            for (uint32_t j = 0; j < HB; ++j)
             {
-                const f4_t other = __builtin_bit_cast(f4_t, in[(h * TB + j) * 64u + lane]);
-                const f4_t mine = kh == 0 ? acc[h][j] : acc[HT + h][j];
+                const f4_t other = __builtin_bit_cast(f4_t, in[(a * HB + j) * 64u + lane]);
+                const f4_t mine = kh == 0 ? acc[a][j] : acc[a][HB + j];
                 const f4_t even = kh == 0 ? mine : other, odd = kh == 0 ? other : mine;
-                finish(keep + h, h, j, even + odd);
+                finish(a, keep + j, even + odd);
             }
     }
 }
@@ -461,12 +505,25 @@ int launch_wide_reduce_norm(opure_dev* dev, const WParams& wp, const float* gain
     return OPURE_OK;
 }
 
+using WIDE_BIG = WideShape<2, 8, 1>;
+
 template <int WF, int AF, int EPI>
 int launch_wide_epi_only(opure_dev* dev, const WParams& wp)
 {
-    OPURE_LAUNCH(dev, (k_gemm_wide<WF, AF, EPI>), dim3(wp.nrg * wp.ncg * wp.splits), dim3(256 * WideDepth<WF>::KH), 0, wp);
-    OPURE_LAUNCH_CHECK("k_gemm_wide");
-    return OPURE_OK;
+    // the kernel shape by the column tiles a workgroup has; every shape sums a
+    // row's blocks in the same order
+    auto go = [&](auto sh) {
+        using SH = decltype(sh);
+        WParams q = wp;
+        q.nrg = (wp.p.tiles + SH::RT - 1u) / SH::RT;
+        OPURE_LAUNCH(dev, (k_gemm_wide<WF, AF, EPI, SH>), dim3(q.nrg * q.ncg * q.splits),
+                     dim3(wide_threads(WF)), 0, q);
+        OPURE_LAUNCH_CHECK("k_gemm_wide");
+        return OPURE_OK;
+    };
+    if (wp.cgs <= 2u) return go(WideShape<1, 2, 1>{});
+    if (wp.cgs <= 4u) return go(WideShape<1, 4, 1>{});
+    return go(WIDE_BIG{});
 }
 
 template <int WF, int AF, int EPI>

@@ -251,7 +251,7 @@ WidePlan wide_plan(const opure_dev* dev, uint32_t wfmt, uint32_t out, uint32_t i
     using namespace opure_gemv;
     WidePlan w;
     const uint32_t KB = kb_of(wfmt);
-    const uint32_t U = wfmt == OPURE_W_I8PC ? WideDepth<OPURE_W_I8PC>::U : WideDepth<OPURE_W_I4G128>::U;
+    const uint32_t U = wfmt == OPURE_W_I8PC ? WideDepth<OPURE_W_I8PC, WIDE_CG>::PU : WideDepth<OPURE_W_I4G128, WIDE_CG>::PU;
     w.tiles = out / 16u;
     w.nblk = in / KB;
     w.mt = (M + 15u) / 16u;

@@ -262,6 +262,32 @@ def test_gemv_wide_matches_reference(dev, case):
             b.free()
 
 
+@pytest.mark.parametrize("case", [(H.W_I8PC, H.A_F16, 80, 320), (H.W_I8PC, H.A_F16, 1168, 64),
+                                  (H.W_I4G128, H.A_F16, 80, 640), (H.W_I4G128, H.A_BF16, 1168, 128),
+                                  (H.W_I4G128, H.A_BF16, 528, 1152)], ids=_ids)
+def test_gemv_wide_shapes_same_rows(dev, case):
+    """The thin GEMM's kernel shapes by row count (up to 32, up to 64, more;
+    one and two column groups, full and ragged last tiles) over weight tiles
+    that do not fill a row group and odd block counts: every row has the bits
+    it has among 256 rows, and those agree with the product in float64."""
+    wfmt, afmt, out, inn = case
+    say("gemv wide shapes", _ids(case))
+    rng = np.random.default_rng(out + inn)
+    lin = O.make_linear(rng, out, inn, wfmt)
+    desc, keep = dev_linear(dev, lin)
+    x_bits, x_f = to_act(rng.standard_normal((256, inn)), afmt)
+    wd = O.dequant(lin, wfmt).astype(np.float64)
+    y = run_gemv(dev, wfmt, desc, x_bits, 256, afmt, H.A_F32, H.EPI_STORE)
+    slack = 4.0 if (wfmt == H.W_I4G128 and afmt == H.A_BF16) else 1.0
+    absref = np.abs(x_f).astype(np.float64) @ np.abs(wd).T
+    assert np.all(np.abs(y - x_f.astype(np.float64) @ wd.T) <= 1e-5 * slack * absref + 1e-6)
+    for M in (17, 31, 32, 33, 48, 64, 65, 127, 128, 129, 145, 255):
+        assert np.array_equal(run_gemv(dev, wfmt, desc, x_bits, M, afmt, H.A_F32, H.EPI_STORE), y[:M]), M
+    for b in keep:
+        if b:
+            b.free()
+
+
 def test_gemv_wide_swiglu(dev):
     wfmt, afmt, out, inn, M = H.W_I8PC, H.A_F16, 16384, 2048, 100
     rng = np.random.default_rng(77)
