@@ -17,7 +17,7 @@
 //  Scores are scaled by attn_scale (1.0 = the reference, which has no
 //  1/sqrt(head_dim): Opure_FlashAttention_Decode.usf:91-104).
 //
-//  fp16/bf16 caches with head_dim 64 or 128 run on matrix cores
+//  fp16/bf16 caches run on matrix cores; head_dim 64 and 128 first
 //  (k_attn_mfma): S^T = K Q^T and O^T = V^T P^T with v_mfma_f32_16x16x32, K
 //  tokens assigned to MFMA rows so that the score tile a lane holds is already
 //  its P^T operand, and V read as V^T tiles straight from the channel-major V
@@ -25,8 +25,10 @@
 //  (22 significant bits), bf16 hi + mid + lo (the fp32 probability to within
 //  2^-25 relative, where one bf16 operand would give 8 bits).  A bf16 model
 //  rounds the attention output to 8 bits next, and any difference from the
-//  exactly summed softmax moves some of those roundings.  fp32 caches and other
-//  head sizes use VALU kernels.
+//  exactly summed softmax moves some of those roundings.  Other head sizes run
+//  on the same kernel with 128-token chunks (32 heads of 96, 4 sequences of 5
+//  rows up to 1,500 tokens: 43.8 us on the VALU, 7.7 us here).  fp32 caches use
+//  VALU kernels.
 // ============================================================================
 #include "internal.h"
 
@@ -769,10 +771,15 @@ __device__ __forceinline__ float merge_val(float sa, float a, float sb, float c)
 // ZS: blockIdx.z holds (sequence, block of 16 * NT query rows) as b * zt + block
 // CL: a workgroup takes the ATTN_GROUP chunks from ATTN_GROUP * blockIdx.y and
 //     writes their merge as partial blockIdx.y
-template <int HD, int AF, int NT, int KK, int NWV, bool ZS, bool CL = false>
+// RH: the head size is p.hd = HD or HD - 16 (every multiple of 16 that is not 64
+//     or 128): channels past it read 0 in K and Q, their V tile is left out
+template <int HD, int AF, int NT, int KK, int NWV, bool ZS, bool CL = false, bool RH = false>
 __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(CL ? 4 : 1))) void k_attn_mfma(AttnParams p)
 {
-    constexpr uint32_t KS = HD / 32u, DT = HD / 16u, EB = 2u, TPW = 32u * KK, OWN = DT * NT / NWV;
+    constexpr uint32_t KS = HD / 32u, DT = HD / 16u, EB = 2u, TPW = 32u * KK, OWN = (DT * NT + NWV - 1u) / NWV;
+    static_assert(!RH || !CL, "the folded kernel is built for head_dim 64");
+    const uint32_t hd = RH ? p.hd : HD;
+    const uint32_t dtn = RH ? hd / 16u : DT;               // channel tiles the head has
     extern __shared__ __align__(16) uint8_t lds_raw[];
     f4_t (*cacc)[DT][NT][64] = reinterpret_cast<f4_t (*)[DT][NT][64]>(lds_raw);
     float (*cml)[NT][16][2] = reinterpret_cast<float (*)[NT][16][2]>(lds_raw + NWV * DT * NT * 64u * 16u);
@@ -818,9 +825,11 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(CL ? 4
         const uint32_t qi = min(qoff + 16u * n + r, Gq - 1u);
         const uint32_t j = qi / group, head = kh * group + (qi - j * group);
         qj[n] = j;
-        const uint8_t* qrow = static_cast<const uint8_t*>(p.q) + ((static_cast<uint64_t>(b * R + j) * p.n_heads + head) * HD) * EB;
+        const uint8_t* qrow = static_cast<const uint8_t*>(p.q) + ((static_cast<uint64_t>(b * R + j) * p.n_heads + head) * hd) * EB;
 #pragma unroll
-        for (uint32_t s = 0; s < KS; ++s) qop[n][s] = *reinterpret_cast<const u4v*>(qrow + (32u * s + 8u * g) * EB);
+        for (uint32_t s = 0; s < KS; ++s)
+            qop[n][s] = !RH || 32u * s + 8u * g < hd ? *reinterpret_cast<const u4v*>(qrow + (32u * s + 8u * g) * EB)
+                                                     : u4v{0u, 0u, 0u, 0u};
     }
     // keeps the loads above issued before the exit below (the compiler would
     // otherwise test the length first and make them wait for it)
@@ -834,7 +843,7 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(CL ? 4
     // the merge's share of wave w: row block w % NT, channel tiles w / NT,
     // w / NT + NWV / NT, ...; the row's last chunk (the folded merge takes
     // chunks up to it) and the merged state of the chunks so far
-    static_assert(NWV % NT == 0 && (DT * NT) % NWV == 0, "whole channel tiles of one row block a wave");
+    static_assert(NWV % NT == 0 && (RH || (DT * NT) % NWV == 0), "whole channel tiles of one row block a wave");
     const uint32_t n_own = wave % NT, qi_own = qoff + 16u * n_own + r;
     const uint32_t last_own = (ctx + min(qi_own, Gq - 1u) / group) / p.chunk;
     float sm = 0.0f, sl = 0.0f;
@@ -882,10 +891,14 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(CL ? 4
                 {
 #pragma unroll
                     for (uint32_t s = 0; s < KS; ++s)
-                        kop[kk][T][s] = pg >= 0 ? *reinterpret_cast<const u4v*>(
-                                                      pool + kv_elem(p.layer, p.n_pages, static_cast<uint32_t>(pg), 0u, p.n_kv, kh,
-                                                                     HD, tok % OPURE_PAGE_SIZE, 32u * s + 8u * g) * EB)
-                                                : u4v{f, f, f, f};
+                    {
+                        const bool in = !RH || 32u * s + 8u * g < hd;
+                        kop[kk][T][s] = pg >= 0 && in ? *reinterpret_cast<const u4v*>(
+                                                            pool + kv_elem(p.layer, p.n_pages, static_cast<uint32_t>(pg), 0u, p.n_kv,
+                                                                           kh, hd, tok % OPURE_PAGE_SIZE, 32u * s + 8u * g) * EB)
+                                        : in          ? u4v{f, f, f, f}
+                                                      : u4v{0u, 0u, 0u, 0u};
+                    }
                 }
             }
             const uint32_t tok = tb + 8u * g;             // 8 tokens of one page
@@ -907,10 +920,10 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(CL ? 4
 #pragma unroll
                 for (uint32_t dt = 0; dt < DT; ++dt)
                 {
-                    if (pg >= 0)
+                    if (pg >= 0 && dt < dtn)
                     {
                         vop[kk][dt] = *reinterpret_cast<const u4v*>(pool + kv_elem(p.layer, p.n_pages, static_cast<uint32_t>(pg), 1u,
-                                                                                   p.n_kv, kh, HD, tok % OPURE_PAGE_SIZE,
+                                                                                   p.n_kv, kh, hd, tok % OPURE_PAGE_SIZE,
                                                                                    16u * dt + r) * EB);
                         if (tok + 8u > total) vop[kk][dt] = mask_tail<AF>(vop[kk][dt], total - tok);   // stale slots read 0
                     }
@@ -1095,7 +1108,7 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(CL ? 4
 #pragma unroll
         for (uint32_t j = 0; j < OWN; ++j)
         {
-            const uint32_t dt = wave / NT + (NWV / NT) * j;
+            const uint32_t dt = RH ? min(wave / NT + (NWV / NT) * j, DT - 1u) : wave / NT + (NWV / NT) * j;
             a[j] = cacc[0][dt][n_own][lane] * ew[0];
 #pragma unroll
             for (int w = 1; w < NWV; ++w)
@@ -1118,8 +1131,11 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(CL ? 4
                 }
 #pragma unroll
                 for (uint32_t j = 0; j < OWN; ++j)
-                    *reinterpret_cast<f4_t*>(p.part_acc + (pbase + qi_own) * HD + 16u * (wave / NT + (NWV / NT) * j) +
-                                             4u * g) = a[j];
+                {
+                    const uint32_t dt = wave / NT + (NWV / NT) * j;
+                    if (!RH || dt < dtn)
+                        *reinterpret_cast<f4_t*>(p.part_acc + (pbase + qi_own) * hd + 16u * dt + 4u * g) = a[j];
+                }
             }
         }
         else
@@ -1335,20 +1351,53 @@ __global__ __launch_bounds__(64) void k_attn_combine(AttnParams p)
     }
 }
 
-template <int HD, int AF, int NT, int KK, int NWV, bool ZS = false, bool CL = false>
+template <int HD, int AF, int NT, int KK, int NWV, bool ZS = false, bool CL = false, bool RH = false>
 int launch_mfma(opure_dev* dev, dim3 grid, const AttnParams& p)
 {
     constexpr uint32_t lds = attn_mfma_lds<HD, NT, NWV>();
     static bool configured = false;
     if (!configured)
     {
-        OPURE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_attn_mfma<HD, AF, NT, KK, NWV, ZS, CL>),
+        OPURE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_attn_mfma<HD, AF, NT, KK, NWV, ZS, CL, RH>),
                                           hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
         configured = true;
     }
-    OPURE_LAUNCH(dev, (k_attn_mfma<HD, AF, NT, KK, NWV, ZS, CL>), grid, dim3(NWV * 64), lds, p);
+    OPURE_LAUNCH(dev, (k_attn_mfma<HD, AF, NT, KK, NWV, ZS, CL, RH>), grid, dim3(NWV * 64), lds, p);
     OPURE_LAUNCH_CHECK("k_attn_mfma");
     return OPURE_OK;
+}
+
+// A 16-bit cache of any other head size, on matrix cores: 128-token chunks
+// (4 waves x 32 tokens), every block of query rows in one launch.  Two
+// 16-row blocks a workgroup up to head_dim 128; past that the output tiles of
+// a second block do not fit beside the K and V operands, so one.
+template <int HDP, int AF>
+int launch_mfma_hd(opure_dev* dev, AttnParams p, uint32_t Gq, uint32_t batch)
+{
+    constexpr int NT2 = HDP <= 128 ? 2 : 1;
+    if (HDP > 32 && HDP % 64 == 0 && Gq <= 16u)
+    {
+        p.zt = 1u;
+        return launch_mfma<HDP, AF, 1, 1, 4, true, false, true>(dev, dim3(p.n_kv, p.nch, batch), p);
+    }
+    p.zt = (Gq + 16u * NT2 - 1u) / (16u * NT2);
+    return launch_mfma<HDP, AF, NT2, 1, 4, true, false, true>(dev, dim3(p.n_kv, p.nch, batch * p.zt), p);
+}
+
+template <int AF>
+int launch_mfma_any(opure_dev* dev, const AttnParams& p, uint32_t Gq, uint32_t batch)
+{
+    switch ((p.hd + 31u) / 32u)
+    {
+    case 1: return launch_mfma_hd<32, AF>(dev, p, Gq, batch);
+    case 2: return launch_mfma_hd<64, AF>(dev, p, Gq, batch);
+    case 3: return launch_mfma_hd<96, AF>(dev, p, Gq, batch);
+    case 4: return launch_mfma_hd<128, AF>(dev, p, Gq, batch);
+    case 5: return launch_mfma_hd<160, AF>(dev, p, Gq, batch);
+    case 6: return launch_mfma_hd<192, AF>(dev, p, Gq, batch);
+    case 7: return launch_mfma_hd<224, AF>(dev, p, Gq, batch);
+    default: return launch_mfma_hd<256, AF>(dev, p, Gq, batch);
+    }
 }
 
 template <int HD, int AF, bool ALL>
@@ -1370,28 +1419,33 @@ int launch_fast(opure_dev* dev, dim3 grid, uint32_t lds, const AttnParams& p)
 
 namespace opure_hip {
 
-// Chunk length of the kernel that runs a shape: 256 for the matrix-core path
-// (fp16/bf16, head_dim 64/128, <= 64 query rows per KV head), 64 for the VALU
-// fast path, 32 for the generic kernel.
-static bool use_mfma(uint32_t hd, uint32_t afmt, uint32_t)
-{
-    return (hd == 64u || hd == 128u) && afmt != OPURE_A_F32;
-}
+// fp16/bf16 caches run on matrix cores at every head size
+static bool use_mfma(uint32_t afmt) { return afmt != OPURE_A_F32; }
+static bool hd_64_128(uint32_t hd) { return hd == 64u || hd == 128u; }
 
 // Chunk length of the kernel that runs a shape: matrix-core path 128 tokens
-// (head_dim 64) or 256 (head_dim 128), VALU fast path 64, generic kernel 32.
-// It depends on the head size and format only, so a row's chunks never
-// depend on how many rows are scored with it.
-uint32_t attn_chunk(uint32_t hd, uint32_t afmt, uint32_t gq)
+// (256 at head_dim 128), fp32 64 (head_dim up to 128) or 32.  It depends on
+// the head size and format only, so a row's chunks never depend on how many
+// rows are scored with it.
+static uint32_t attn_chunk(uint32_t hd, uint32_t afmt)
 {
-    if (use_mfma(hd, afmt, gq)) return hd == 64u ? 128u : 256u;
+    if (use_mfma(afmt)) return hd == 128u ? 256u : 128u;
     return hd <= 128u ? 64u : 32u;
+}
+
+// The chunk length that bounds max_ctx: a head size other than 64 and 128
+// takes the same contexts (and, below, the same query rows) in every format,
+// those of the fp32 kernels.
+static uint32_t limit_chunk(uint32_t hd, uint32_t afmt)
+{
+    return hd_64_128(hd) ? attn_chunk(hd, afmt) : (hd <= 128u ? 64u : 32u);
 }
 
 uint64_t attn_partial_bytes(uint32_t batch, uint32_t n_kv, uint32_t group, uint32_t rows, uint32_t hd, uint32_t afmt,
                             uint32_t max_ctx)
 {
-    const uint32_t ch = attn_chunk(hd, afmt, group * rows);
+    // the shorter chunks: a cache off 16-byte alignment takes the generic kernel
+    const uint32_t ch = limit_chunk(hd, afmt);
     const uint32_t nch = (max_ctx + ch - 1u) / ch;
     const uint64_t q = static_cast<uint64_t>(batch) * n_kv * nch * group * rows;
     return align_up(q * hd * 4u, 256) + align_up(q * 2u * 4u, 256);
@@ -1415,10 +1469,10 @@ int attn_validate(const opure_model* m, const opure_kv* kv, uint32_t batch, uint
                   "attention: max_ctx %u beyond the page-table capacity %u", max_ctx,
                   kv->max_pages_per_seq * OPURE_PAGE_SIZE);
     OPURE_REQUIRE(m->afmt <= OPURE_A_BF16, OPURE_E_INVALID, "attention: bad activation format");
-    const uint32_t group = m->n_heads / m->n_kv_heads, CH = attn_chunk(m->head_dim, m->afmt, group * rows);
+    const uint32_t group = m->n_heads / m->n_kv_heads, CH = limit_chunk(m->head_dim, m->afmt);
     OPURE_REQUIRE((max_ctx + CH - 1u) / CH <= 1024u, OPURE_E_CAPACITY, "attention: max_ctx %u has more than 1024 chunks",
                   max_ctx);
-    if (!use_mfma(m->head_dim, m->afmt, group * rows))
+    if (!use_mfma(m->afmt) || !hd_64_128(m->head_dim))
     {
         // VALU kernels hold the query rows (and, generic, the scores and K/V) in LDS
         const uint64_t eb = act_bytes(m->afmt), hd = m->head_dim;
@@ -1450,7 +1504,11 @@ int attn_launch(opure_dev* dev, const opure_model* m, const opure_kv* kv, uint32
     p.max_pages = kv->max_pages_per_seq;
     p.layer = layer;
     const uint32_t group = m->n_heads / m->n_kv_heads, Gq = group * rows;
-    p.chunk = attn_chunk(m->head_dim, m->afmt, Gq);
+    // the matrix-core kernel reads 16 bytes a lane; at head sizes other than 64
+    // and 128 a cache or Q off that alignment takes the generic kernel
+    const bool aligned = ((reinterpret_cast<uintptr_t>(kv->pool) | reinterpret_cast<uintptr_t>(q)) & 15u) == 0u;
+    const bool mfma = use_mfma(m->afmt) && (hd_64_128(m->head_dim) || aligned);
+    p.chunk = mfma ? attn_chunk(m->head_dim, m->afmt) : limit_chunk(m->head_dim, m->afmt);
     p.nch = (max_ctx + p.chunk - 1u) / p.chunk;
     p.afmt = m->afmt;
     p.scale = m->attn_scale;
@@ -1466,8 +1524,14 @@ int attn_launch(opure_dev* dev, const opure_model* m, const opure_kv* kv, uint32
     // head_dim 64 on matrix cores: the combine merges groups of ATTN_GROUP
     // chunks as the folded kernel does (1 item = 1 group), unless the folded
     // kernel wrote the groups' partials itself
-    uint32_t grp = use_mfma(hd, p.afmt, Gq) && hd == 64u ? ATTN_GROUP : 1u;
-    if (use_mfma(hd, p.afmt, Gq))
+    uint32_t grp = mfma && hd == 64u ? ATTN_GROUP : 1u;
+    if (mfma && !hd_64_128(hd))
+    {
+        const int rc = p.afmt == OPURE_A_F16 ? launch_mfma_any<OPURE_A_F16>(dev, p, Gq, batch)
+                                             : launch_mfma_any<OPURE_A_BF16>(dev, p, Gq, batch);
+        if (rc) return rc;
+    }
+    else if (mfma)
     {
         // head_dim 64 on a grid of few workgroups (the 1B shape at batch 1:
         // 136 -> 272 workgroups): one 16-row block of query rows a
@@ -1534,9 +1598,7 @@ int attn_launch(opure_dev* dev, const opure_model* m, const opure_kv* kv, uint32
         // a short context at head_dim 64: a workgroup a pair of query rows, a
         // wave a chunk, merged in the workgroup (no combine launch)
         const dim3 g(p.n_kv, (Gq + 1u) / 2u, batch), blk(64u * p.nch);
-        if (p.afmt == OPURE_A_F32) OPURE_LAUNCH(dev, k_attn_split<OPURE_A_F32>, g, blk, 0, p);
-        else if (p.afmt == OPURE_A_F16) OPURE_LAUNCH(dev, k_attn_split<OPURE_A_F16>, g, blk, 0, p);
-        else OPURE_LAUNCH(dev, k_attn_split<OPURE_A_BF16>, g, blk, 0, p);
+        OPURE_LAUNCH(dev, k_attn_split<OPURE_A_F32>, g, blk, 0, p);
         OPURE_LAUNCH_CHECK("k_attn_split");
         return OPURE_OK;
     }
@@ -1549,15 +1611,8 @@ int attn_launch(opure_dev* dev, const opure_model* m, const opure_kv* kv, uint32
         const uint32_t lds = all ? static_cast<uint32_t>(all_lds) : Gq * hd * 4u;
         const dim3 g = all ? dim3(p.n_kv, 1u, batch) : grid;
         int rc;
-        if (hd == 64u && p.afmt == OPURE_A_F32) rc = launch_fast<64, OPURE_A_F32, false>(dev, g, lds, p);
-        else if (hd == 64u && p.afmt == OPURE_A_F16) rc = launch_fast<64, OPURE_A_F16, false>(dev, g, lds, p);
-        else if (hd == 64u) rc = launch_fast<64, OPURE_A_BF16, false>(dev, g, lds, p);
-        else if (p.afmt == OPURE_A_F32)
-            rc = all ? launch_fast<128, OPURE_A_F32, true>(dev, g, lds, p) : launch_fast<128, OPURE_A_F32, false>(dev, g, lds, p);
-        else if (p.afmt == OPURE_A_F16)
-            rc = all ? launch_fast<128, OPURE_A_F16, true>(dev, g, lds, p) : launch_fast<128, OPURE_A_F16, false>(dev, g, lds, p);
-        else
-            rc = all ? launch_fast<128, OPURE_A_BF16, true>(dev, g, lds, p) : launch_fast<128, OPURE_A_BF16, false>(dev, g, lds, p);
+        if (hd == 64u) rc = launch_fast<64, OPURE_A_F32, false>(dev, g, lds, p);
+        else rc = all ? launch_fast<128, OPURE_A_F32, true>(dev, g, lds, p) : launch_fast<128, OPURE_A_F32, false>(dev, g, lds, p);
         if (rc) return rc;
         if (all) return OPURE_OK;
     }

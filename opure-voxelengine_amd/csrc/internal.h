@@ -245,7 +245,6 @@ bool gemv_is_wave_per_tile(const opure_dev* dev, const GemvCall& c);
 uint32_t tiled_block_k(uint32_t wfmt);      // k values per 64-byte block
 
 // ---- attention (attention.hip) ---------------------------------------------
-uint32_t attn_chunk(uint32_t head_dim, uint32_t afmt, uint32_t query_rows_per_kv_head);
 uint64_t attn_partial_bytes(uint32_t batch, uint32_t n_kv, uint32_t group, uint32_t rows, uint32_t hd, uint32_t afmt,
                             uint32_t max_ctx);
 int      attn_validate(const opure_model* m, const opure_kv* kv, uint32_t batch, uint32_t rows, uint32_t max_ctx);

@@ -571,6 +571,59 @@ def test_attention_paged_matches_oracle(dev, case):
         assert np.array_equal(one[0], got[j])
 
 
+@pytest.mark.parametrize("hd", [16, 32, 48, 80, 96, 112, 144, 160, 176, 192, 208, 224, 240, 256])
+@pytest.mark.parametrize("afmt", [H.A_F16, H.A_BF16], ids=["f16", "bf16"])
+def test_attention_every_head_size(dev, afmt, hd):
+    """16-bit caches of every head size but 64 and 128 on matrix cores: 21
+    query rows a KV head (blocks of 16 and 32 rows, a ragged last one), contexts
+    that end on either side of a 128-token chunk, stale NaN slots past the end;
+    within one storage ulp of the softmax in float64, row j equal to a one-row
+    call at its position; the same cache off 16-byte alignment (the generic
+    kernel) agrees to a storage ulp."""
+    say("attention head size", hd, afmt)
+    rng = np.random.default_rng(hd + afmt)
+    nh, nkv, R, ctx = 14, 2, 3, [0, 126, 125, 257, 390]
+    B, mp = len(ctx), 26
+    pool_bits, pool_f = to_act(rng.standard_normal((1, B * mp, 2, nkv, 16 * hd)), afmt)
+    pt = rng.permutation(B * mp).reshape(B, mp).astype(np.int32)
+    K = pool_f[0, :, 0].reshape(-1, nkv, 16, hd)
+    V = pool_f[0, :, 1].reshape(-1, nkv, hd, 16).transpose(0, 1, 3, 2)
+    q_bits, q_f = to_act(rng.standard_normal((B * R, nh * hd)), afmt)
+    ref = np.zeros((B * R, nh, hd))
+    nan = 0x7E00 if afmt == H.A_F16 else 0x7FC0
+    planes_k, planes_v = pool_bits[0, :, 0].reshape(-1, nkv, 16, hd), pool_bits[0, :, 1].reshape(-1, nkv, hd, 16)
+    for b, c in enumerate(ctx):
+        k = K[pt[b]].transpose(0, 2, 1, 3).reshape(-1, nkv, hd).astype(np.float64)
+        v = V[pt[b]].transpose(0, 2, 1, 3).reshape(-1, nkv, hd).astype(np.float64)
+        for j in range(R):
+            for h in range(nh):
+                s = k[:c + j + 1, h // 7] @ q_f[b * R + j].reshape(nh, hd)[h].astype(np.float64) * hd ** -0.5
+                w = np.exp(s - s.max())
+                ref[b * R + j, h] = w @ v[:c + j + 1, h // 7] / w.sum()
+        last, slot = pt[b, (c + R - 1) // 16], (c + R - 1) % 16 + 1
+        planes_k[last, :, slot:] = nan
+        planes_v[last, :, :, slot:] = nan
+    m = attn_model(nh, nkv, hd, afmt, hd ** -0.5)
+    got = run_attn(dev, m, pool_bits, pt, ctx, R, q_bits)
+    want = to_act(ref.reshape(B * R, -1), afmt)[1]
+    ulp = 2.0 ** -10 if afmt == H.A_F16 else 2.0 ** -7
+    assert (np.abs(from_act(got, afmt) - want) <= ulp * np.abs(want) + 2e-6).all()
+    for b in (1, 4):
+        for j in range(R):
+            one = run_attn(dev, m, pool_bits, pt[b:b + 1], [ctx[b] + j], 1, q_bits[b * R + j:b * R + j + 1])
+            assert np.array_equal(one[0], got[b * R + j])
+    pb = dev.upload(np.concatenate([np.zeros(1, np.uint16), pool_bits.ravel()]))
+    ptb, sl, qb = dev.upload(pt), dev.upload(np.asarray(ctx, np.int32)), dev.upload(q_bits)
+    ob = dev.alloc(q_bits.nbytes)
+    kv = H.KV(int(pb) + 2, B * mp, 16, int(ptb), mp)
+    a = H.AttnArgs(C.pointer(m), C.pointer(kv), 0, B, R, int(sl), max(ctx) + R, int(qb), int(ob))
+    H.check(H.lib().opure_attn_decode_paged(dev.h, C.byref(a)))
+    dev.sync()
+    assert (np.abs(from_act(dev.download(ob, np.uint16, q_bits.shape), afmt) - want) <= ulp * np.abs(want) + 2e-6).all()
+    for x in (pb, ptb, sl, qb, ob):
+        x.free()
+
+
 # fp32 launches over few chunks of 64 tokens: head_dim, query heads, KV heads,
 # rows, contexts (rows ending on either side of chunk boundaries)
 FAST_ALL_CASES = [
