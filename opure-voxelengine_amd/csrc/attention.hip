@@ -1199,8 +1199,8 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(CL ? 4
 // denominator with a fixed butterfly), then channels d = lane + 64 i
 // (i < DPL), summing the items' outputs in order.  The first CB partials'
 // outputs are loaded together with the statistics, so a context of up to CB
-// partials costs one round trip (CB 20 where a launch has at most 20
-// partials: fewer loads of the clamped last one).
+// partials costs one round trip (CB 8 or 20 where a launch has at most that
+// many: fewer loads of the clamped last one).
 template <int DPL, int GRP, uint32_t CB = 32u>
 __global__ __launch_bounds__(64) void k_attn_combine(AttnParams p)
 {
@@ -1567,6 +1567,20 @@ int attn_launch(opure_dev* dev, const opure_model* m, const opure_kv* kv, uint32
                 p.cpp = ATTN_GROUP;
                 grp = 1u;
             }
+            // head_dim 128 over more than 32 query rows (a prompt's parts): the
+            // 32-row blocks along z of one launch -- a launch a block ended in a
+            // last wave of workgroups each (640 on 512 slots)
+            if (hd == 128u && Gq > 32u && batch * ((Gq + 31u) / 32u) <= 65535u)
+            {
+                AttnParams pq = p;
+                pq.qoff = 0u;
+                pq.zt = (Gq + 31u) / 32u;
+                const dim3 g(p.n_kv, p.nch, batch * pq.zt);
+                const int rc = p.afmt == OPURE_A_F16 ? launch_mfma<128, OPURE_A_F16, 2, 2, 4, true>(dev, g, pq)
+                                                     : launch_mfma<128, OPURE_A_BF16, 2, 2, 4, true>(dev, g, pq);
+                if (rc) return rc;
+            }
+            else
             for (uint32_t q0 = 0; q0 < Gq; q0 += 32u)
             {
                 AttnParams pq = p;
@@ -1630,19 +1644,22 @@ int attn_launch(opure_dev* dev, const opure_model* m, const opure_kv* kv, uint32
         OPURE_LAUNCH_CHECK("k_attn_chunk_generic");
     }
     const dim3 cgrid(p.n_heads, batch * rows);
-    const bool few = p.npart <= 20u;
-    if (grp > 1u && few) OPURE_LAUNCH(dev, (k_attn_combine<1, ATTN_GROUP, 20u>), cgrid, dim3(64), 0, p);
-    else if (grp > 1u) OPURE_LAUNCH(dev, (k_attn_combine<1, ATTN_GROUP>), cgrid, dim3(64), 0, p);
+    // outputs preloaded: as many as the launch has partials, of three sizes (a
+    // load of the clamped last partial costs as much as one that is used: 256
+    // rows of 32 heads of 128 with 5 partials CMB0 us at 32, CMB1 at 8)
+    auto combine = [&](auto few, auto some, auto many) {
+        auto* k = p.npart <= 8u ? few : p.npart <= 20u ? some : many;
+        OPURE_LAUNCH(dev, k, cgrid, dim3(64), 0, p);
+    };
+    if (grp > 1u)
+        combine(&k_attn_combine<1, ATTN_GROUP, 8u>, &k_attn_combine<1, ATTN_GROUP, 20u>, &k_attn_combine<1, ATTN_GROUP, 32u>);
     else
         switch ((p.hd + 63u) / 64u)
         {
-        case 1:
-            if (few) OPURE_LAUNCH(dev, (k_attn_combine<1, 1, 20u>), cgrid, dim3(64), 0, p);
-            else OPURE_LAUNCH(dev, (k_attn_combine<1, 1>), cgrid, dim3(64), 0, p);
-            break;
-        case 2: OPURE_LAUNCH(dev, (k_attn_combine<2, 1>), cgrid, dim3(64), 0, p); break;
-        case 3: OPURE_LAUNCH(dev, (k_attn_combine<3, 1>), cgrid, dim3(64), 0, p); break;
-        default: OPURE_LAUNCH(dev, (k_attn_combine<4, 1>), cgrid, dim3(64), 0, p); break;
+        case 1: combine(&k_attn_combine<1, 1, 8u>, &k_attn_combine<1, 1, 20u>, &k_attn_combine<1, 1, 32u>); break;
+        case 2: combine(&k_attn_combine<2, 1, 8u>, &k_attn_combine<2, 1, 20u>, &k_attn_combine<2, 1, 32u>); break;
+        case 3: combine(&k_attn_combine<3, 1, 8u>, &k_attn_combine<3, 1, 20u>, &k_attn_combine<3, 1, 32u>); break;
+        default: combine(&k_attn_combine<4, 1, 8u>, &k_attn_combine<4, 1, 20u>, &k_attn_combine<4, 1, 32u>); break;
         }
     OPURE_LAUNCH_CHECK("k_attn_combine");
     return OPURE_OK;
