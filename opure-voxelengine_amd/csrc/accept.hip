@@ -1346,6 +1346,139 @@ __global__ __launch_bounds__(NT) void k_sample_sliced(SampleParams p)
     }
 }
 
+// ---- greedy acceptance over stored logits in one launch -------------------------
+// Grid (slices, R, B): a workgroup takes the argmax of a slice of one row and
+// publishes it as two tagged words (the sampler's slots and launch counts: a
+// row's count tags its words, so both kernels may share them); the last
+// workgroup of a sequence gathers its R rows, accepts, rolls back and moves the
+// rows' counts on.  Only that workgroup waits, for workgroups dispatched before
+// it, and the wait is bounded.  Bound by reading the logits: 96 rows of 128,256
+// 24.8 us as two launches (scalar loads, then an acceptance launch of 8.3 us
+// over the partials), 14.3 here.
+struct GreedySlicedParams {
+    const float* logits;
+    uint32_t V, slices;
+    uint32_t* epoch;
+    uint64_t* slots;
+    uint32_t wait_limit;
+    uint32_t* err;
+    GreedyParams g;
+};
+
+__global__ __launch_bounds__(NT) void k_greedy_sliced(GreedySlicedParams p)
+{
+    typedef float f4v __attribute__((ext_vector_type(4)));
+    __shared__ float sv[NT / 64];
+    __shared__ int32_t si[NT / 64];
+    __shared__ int32_t am[64], sdraft[64];
+    __shared__ uint32_t stag[64], s_n;
+    __shared__ RollbackPre pre;
+    const uint32_t sl = blockIdx.x, y = blockIdx.y, b = blockIdx.z, R = gridDim.y, V = p.V, t = threadIdx.x;
+    const uint32_t r = b * R + y, wave = t >> 6, lane = t & 63u;
+    const float* row = p.logits + static_cast<uint64_t>(r) * V;
+    uint64_t* slots = p.slots + static_cast<uint64_t>(b) * R * REJ_MAX_SLICES * 3u;
+    const uint32_t epoch = t == 0u ? __hip_atomic_load(p.epoch + r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+    const uint32_t v0 = sl * SLICE;
+    // the quads v0 + 4 (i NT + t), as k_sample_sliced loads them
+    float x[PER];
+    const bool vec = (V & 3u) == 0u && (reinterpret_cast<uintptr_t>(p.logits) & 15u) == 0u;
+#pragma unroll
+    for (uint32_t i = 0; i < PER / 4u; ++i)
+    {
+        const uint32_t v = v0 + 4u * (i * NT + t);
+        if (vec)
+        {
+            const f4v q = *reinterpret_cast<const f4v*>(row + min(v, V - 4u));
+#pragma unroll
+            for (uint32_t e = 0; e < 4u; ++e) x[4u * i + e] = q[e];
+        }
+        else
+        {
+#pragma unroll
+            for (uint32_t e = 0; e < 4u; ++e) x[4u * i + e] = row[min(v + e, V - 1u)];
+        }
+    }
+    float bv = -__builtin_huge_valf();
+    int32_t bi = 0x7FFFFFFF;
+#pragma unroll
+    for (uint32_t i = 0; i < PER; ++i)
+    {
+        const uint32_t v = v0 + 4u * ((i / 4u) * NT + t) + (i & 3u);
+        const float c = x[i] != x[i] ? -__builtin_huge_valf() : x[i];
+        if (v < V && (c > bv || (c == bv && static_cast<int32_t>(v) < bi))) { bv = c; bi = static_cast<int32_t>(v); }
+    }
+    auto wave_best = [&]() {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1)
+        {
+            const float ov = __shfl_xor(bv, o);
+            const int32_t oi = __shfl_xor(bi, o);
+            if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
+        }
+    };
+    wave_best();
+    if (lane == 0u) { sv[wave] = bv; si[wave] = bi; }
+    __syncthreads();
+    if (t == 0u)
+    {
+#pragma unroll
+        for (uint32_t w = 1; w < NT / 64u; ++w)
+            if (sv[w] > bv || (sv[w] == bv && si[w] < bi)) { bv = sv[w]; bi = si[w]; }
+        uint64_t* mine = slots + (static_cast<uint64_t>(y) * REJ_MAX_SLICES + sl) * 3u;
+        slot_put(mine, slot_f32(epoch + 1u, bv));
+        slot_put(mine + 1, slot_f32(epoch + 1u, __int_as_float(bi)));
+    }
+    if (sl + 1u != p.slices || y + 1u != R) return;       // not the sequence's last workgroup
+
+    const GreedyParams& g = p.g;
+    if (t < g.K) sdraft[t] = g.drafts[static_cast<uint64_t>(b) * g.drafts_stride + t];
+    if (g.rollback && t == 64u) pre = rollback_pre(g.rb, b);
+    if (t < R) stag[t] = __hip_atomic_load(p.epoch + b * R + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+    __syncthreads();
+    // a wave a row, a lane a slice
+    for (uint32_t q = wave; q < R; q += NT / 64u)
+    {
+        const uint32_t tag = stag[q];
+        uint64_t* w = slots + (static_cast<uint64_t>(q) * REJ_MAX_SLICES + lane) * 3u;
+        uint64_t wv = 0, wi = 0;
+        for (uint32_t n = 0;; ++n)
+        {
+            bool ok = true;
+            if (lane < p.slices)
+            {
+                wv = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                wi = __hip_atomic_load(w + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                ok = (wv >> 32) == tag && (wi >> 32) == tag;
+            }
+            if (__all(ok)) break;
+            if (n >= p.wait_limit)
+            {
+                if (lane == 0u) p.err[ERR_WAIT] = 1u;
+                break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+        }
+        bv = lane < p.slices ? __uint_as_float(static_cast<uint32_t>(wv)) : -__builtin_huge_valf();
+        bi = lane < p.slices ? static_cast<int32_t>(static_cast<uint32_t>(wi)) : 0x7FFFFFFF;
+        wave_best();
+        if (lane == 0u) am[q] = bi == 0x7FFFFFFF ? 0 : bi;
+    }
+    __syncthreads();
+    // every workgroup of the sequence has read its row's count
+    if (t < R) __hip_atomic_store(p.epoch + b * R + t, stag[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (t == 0u)
+    {
+        uint32_t n = 0;
+        while (n < g.K && am[n] == sdraft[n]) ++n;
+        s_n = n;
+    }
+    __syncthreads();
+    const uint32_t n = s_n;
+    if (t < R) g.out_tokens[b * R + t] = t < n ? sdraft[t] : (t == n ? am[n] : -1);
+    if (t == 0u) g.accepted[b] = static_cast<int32_t>(n);
+    if (g.rollback) rollback_seq(g.rb, b, n, pre);
+}
+
 // vocabularies past REJ_MAX_SLICES slices: one workgroup a row
 __global__ __launch_bounds__(256) void k_sample(SampleParams p)
 {
@@ -1454,8 +1587,8 @@ int greedy_from_partials(opure_dev* dev, const float* am_val, const int32_t* am_
     return OPURE_OK;
 }
 
-int argmax_partials_launch(opure_dev* dev, const float* logits, uint32_t rows, uint32_t V, float* am_val,
-                           int32_t* am_idx)
+static int argmax_partials_launch(opure_dev* dev, const float* logits, uint32_t rows, uint32_t V, float* am_val,
+                                  int32_t* am_idx)
 {
     ArgmaxParams ap;
     ap.logits = logits;
@@ -1470,15 +1603,53 @@ int argmax_partials_launch(opure_dev* dev, const float* logits, uint32_t rows, u
     return OPURE_OK;
 }
 
-int accept_greedy_launch(opure_dev* dev, const opure_accept_args* a, void* ws)
+// the sliced kernels' launch counts and slots
+static void smp_sync(const opure_dev* dev, uint32_t*& epoch, uint64_t*& slots)
+{
+    uint8_t* sync = static_cast<uint8_t*>(dev->rej_sync) + REJ_SYNC_BYTES - SMP_SYNC_BYTES;
+    epoch = reinterpret_cast<uint32_t*>(sync);
+    slots = reinterpret_cast<uint64_t*>(sync + SMP_SYNC_ROWS * sizeof(uint32_t));
+}
+
+int greedy_from_logits(opure_dev* dev, const float* logits, uint32_t V, float* am_val, int32_t* am_idx, uint32_t batch,
+                       uint32_t K, const int32_t* drafts, uint32_t stride, int32_t* out_tokens, int32_t* accepted,
+                       const opure_rollback_args* rb)
+{
+    const uint32_t rows = batch * (K + 1u);
+    // one launch where the rows and their slices have slots; past that the
+    // argmax partials and the acceptance are two
+    if (!dev->rej_sync || !dev->err || static_cast<uint64_t>(batch) * (K + 1u) > SMP_SYNC_ROWS || rej_slices(V) > REJ_MAX_SLICES)
+    {
+        const int rc = argmax_partials_launch(dev, logits, rows, V, am_val, am_idx);
+        if (rc) return rc;
+        return greedy_from_partials(dev, am_val, am_idx, argmax_parts(V), batch, K, drafts, stride, out_tokens, accepted, rb);
+    }
+    GreedySlicedParams p{};
+    p.logits = logits;
+    p.V = V;
+    p.slices = rej_slices(V);
+    smp_sync(dev, p.epoch, p.slots);
+    p.wait_limit = dev->wait_limit;
+    p.err = dev->err;
+    p.g.K = K;
+    p.g.drafts = drafts;
+    p.g.drafts_stride = stride;
+    p.g.out_tokens = out_tokens;
+    p.g.accepted = accepted;
+    p.g.rollback = rb ? 1u : 0u;
+    if (rb) p.g.rb = rollback_params(rb);
+    OPURE_LAUNCH(dev, k_greedy_sliced, dim3(p.slices, K + 1u, batch), dim3(NT), 0, p);
+    OPURE_LAUNCH_CHECK("k_greedy_sliced");
+    return OPURE_OK;
+}
+
+static int accept_greedy_launch(opure_dev* dev, const opure_accept_args* a, void* ws)
 {
     const uint32_t rows = a->batch * (a->k + 1u), parts = argmax_parts(a->vocab);
     float* am_val = static_cast<float*>(ws);
     int32_t* am_idx = reinterpret_cast<int32_t*>(static_cast<char*>(ws) + align_up(static_cast<uint64_t>(parts) * rows * 4u, 256));
-    const int rc = argmax_partials_launch(dev, a->target_logits, rows, a->vocab, am_val, am_idx);
-    if (rc) return rc;
-    return greedy_from_partials(dev, am_val, am_idx, parts, a->batch, a->k, a->drafts, a->drafts_stride,
-                                a->out_tokens, a->accepted, nullptr);
+    return greedy_from_logits(dev, a->target_logits, a->vocab, am_val, am_idx, a->batch, a->k, a->drafts, a->drafts_stride,
+                              a->out_tokens, a->accepted, nullptr);
 }
 
 int accept_rejection_launch(opure_dev* dev, const opure_accept_args* a, void* ws, const int32_t* seq_len,
@@ -1681,9 +1852,7 @@ int opure_sample_rows(opure_dev* dev, const opure_sample_args* a)
         OPURE_LAUNCH_CHECK("k_sample");
         return OPURE_OK;
     }
-    uint8_t* sync = static_cast<uint8_t*>(dev->rej_sync) + REJ_SYNC_BYTES - SMP_SYNC_BYTES;
-    s.epoch = reinterpret_cast<uint32_t*>(sync);
-    s.slots = reinterpret_cast<uint64_t*>(sync + SMP_SYNC_ROWS * sizeof(uint32_t));
+    smp_sync(dev, s.epoch, s.slots);
     s.wait_limit = dev->wait_limit;
     s.err = dev->err;
     for (uint32_t r0 = 0; r0 < a->rows; r0 += SMP_SYNC_ROWS)

@@ -16,7 +16,7 @@
 //  Host side: device object, errors, workspace
 // ---------------------------------------------------------------------------
 constexpr uint32_t REJ_SYNC_SEQS = 4096;
-// the sliced sampler's state: a launch count a row, then [SMP_SYNC_ROWS][64
+// the sliced sampler's and greedy acceptance's state: a launch count a row, then [SMP_SYNC_ROWS][64
 // slices][3] tagged words; at the end of the rejection sampler's
 constexpr uint32_t SMP_SYNC_ROWS = 4096;
 constexpr uint64_t SMP_SYNC_BYTES = SMP_SYNC_ROWS * 4ull + SMP_SYNC_ROWS * 64ull * 3ull * 8ull;
@@ -260,10 +260,10 @@ RollbackParams rollback_params(const opure_rollback_args* a);
 int      greedy_from_partials(opure_dev* dev, const float* am_val, const int32_t* am_idx, uint32_t parts,
                               uint32_t batch, uint32_t K, const int32_t* drafts, uint32_t stride, int32_t* out_tokens,
                               int32_t* accepted, const opure_rollback_args* rb);
-int      accept_greedy_launch(opure_dev* dev, const opure_accept_args* a, void* ws);
-// per-4096-column (value, lowest index) argmax partials [parts][rows] of fp32 logits
-int      argmax_partials_launch(opure_dev* dev, const float* logits, uint32_t rows, uint32_t V, float* am_val,
-                                int32_t* am_idx);
+// the same over stored logits (am_val, am_idx: room for argmax_parts(V) partials a row)
+int      greedy_from_logits(opure_dev* dev, const float* logits, uint32_t V, float* am_val, int32_t* am_idx,
+                            uint32_t batch, uint32_t K, const int32_t* drafts, uint32_t stride, int32_t* out_tokens,
+                            int32_t* accepted, const opure_rollback_args* rb);
 int      accept_rejection_launch(opure_dev* dev, const opure_accept_args* a, void* ws, const int32_t* seq_len,
                                  int32_t* new_seq_len);
 int      rollback_validate(const opure_rollback_args* a);

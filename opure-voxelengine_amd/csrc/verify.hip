@@ -483,18 +483,12 @@ int opure_verify_step(opure_dev* dev, const opure_verify_args* a)
     if (a->accept_mode == OPURE_ACCEPT_GREEDY && !fused)
     {
         // greedy acceptance and the rollback run in one kernel
-        uint32_t parts = 0;
         if (wide)
-        {
-            parts = argmax_parts(m->vocab);
-            if ((rc = argmax_partials_launch(dev, a->logits, MR, m->vocab, c.logits.am_val, c.logits.am_idx))) return rc;
-        }
+            rc = greedy_from_logits(dev, a->logits, m->vocab, c.logits.am_val, c.logits.am_idx, B, R - 1u, a->tokens + 1, R,
+                                    a->out_tokens, a->accepted, a->rollback ? &rb : nullptr);
         else
-        {
-            parts = gemv_grid(dev, c);
-        }
-        rc = greedy_from_partials(dev, c.logits.am_val, c.logits.am_idx, parts, B, R - 1u, a->tokens + 1, R,
-                                  a->out_tokens, a->accepted, a->rollback ? &rb : nullptr);
+            rc = greedy_from_partials(dev, c.logits.am_val, c.logits.am_idx, gemv_grid(dev, c), B, R - 1u, a->tokens + 1, R,
+                                      a->out_tokens, a->accepted, a->rollback ? &rb : nullptr);
         if (rc) return rc;
     }
     else if (a->accept_mode == OPURE_ACCEPT_REJECTION)

@@ -747,6 +747,43 @@ def test_accept_greedy_bit_exact(dev):
     assert np.array_equal(acc, w_acc) and np.array_equal(out, w_out)
 
 
+@pytest.mark.parametrize("B,K,V,off", [(1, 0, 1, 0), (3, 2, 7, 1), (2, 5, 4095, 0), (5, 4, 4097, 0), (4, 63, 8192, 0),
+                                       (2, 1, 262144, 0), (2, 1, 262145, 0), (600, 7, 100, 0)], ids=lambda v: str(v))
+def test_accept_greedy_slices_bit_exact(dev, B, K, V, off):
+    """One slice, whole slices, a remainder, the most slices and one past them
+    (two launches), 64 rows a sequence, more rows than there are slots; ties
+    (also of 0 and -0), NaN and all -inf rows, logits off 16-byte alignment.
+    Twice, so the words carry two launch counts, with a sampling launch (which
+    shares the rows' counts) between."""
+    say("greedy slices", B, K, V, off)
+    rng = np.random.default_rng(B + K + V)
+    lg = rng.integers(-3, 4, (B, K + 1, V)).astype(np.float32)
+    lg[lg == 0] *= rng.choice([1.0, -1.0], int((lg == 0).sum())).astype(np.float32)
+    lg[0, 0, V // 2] = np.nan
+    if B > 1:
+        lg[1, 0] = -np.inf
+        lg[-1, -1] = np.nan
+    c = np.where(np.isnan(lg), -np.inf, lg)
+    drafts = np.zeros((B, K), np.int32)
+    for b in range(B):
+        drafts[b] = c[b, :K].argmax(1)
+        if K:
+            drafts[b, min(K - 1, b % (K + 1))] += b % (K + 1) < K
+    buf = dev.upload(np.concatenate([np.zeros(off, np.float32), lg.ravel()]))
+    db = dev.upload(drafts) if K else dev.alloc(4)
+    ot, ac = dev.alloc(B * (K + 1) * 4), dev.alloc(B * 4)
+    pos, sq, so = (dev.upload(np.zeros(3, np.uint32)) for _ in range(3))
+    w_out, w_acc = O.accept_greedy(lg, drafts)
+    a = H.AcceptArgs(B, K, V, int(buf) + 4 * off, None, int(db), K, 1.0, 0, None, int(ot), int(ac), None)
+    for _ in range(2):
+        H.check(H.lib().opure_accept_greedy(dev.h, C.byref(a)))
+        s = H.SampleArgs(min(3, B * (K + 1)), V, int(buf) + 4 * off, 1.0, 1, int(pos), int(sq), 0, int(so))
+        H.check(H.lib().opure_sample_rows(dev.h, C.byref(s)))
+        dev.sync()
+        assert np.array_equal(dev.download(ac, np.int32, (B,)), w_acc)
+        assert np.array_equal(dev.download(ot, np.int32, (B, K + 1)), w_out)
+
+
 def test_attention_folded_grid_same_bits(dev):
     """A batch big enough that the launch folds two chunks into a workgroup
     (head_dim 64, 16 sequences of up to 9000 tokens) gives every sequence
