@@ -366,6 +366,28 @@ int opure_verify_reserve(opure_dev* dev, const opure_model* model, uint32_t batc
                          uint32_t max_ctx);
 int opure_verify_step(opure_dev* dev, const opure_verify_args* a);
 
+/* ---- prompt step: `rows` tokens of ONE sequence (kv's first page-table row)
+ *      at positions seq_len[0] .. seq_len[0] + rows - 1 through the layers,
+ *      their K/V appended; with `logits`, the last row's logits and (out_token)
+ *      their argmax.  A prefill: the verify step with logits == NULL does the
+ *      same for up to OPURE_MAX_BATCH_ROWS rows.  Quantised weights, 16-bit activations, head_dim 64 or 128,
+ *      OPURE_MAX_ROWS + 1 .. OPURE_MAX_PROMPT_ROWS rows. */
+#define OPURE_MAX_PROMPT_ROWS 2048
+typedef struct opure_prompt_args {
+    const opure_model* model;
+    const opure_kv*    kv;
+    const int32_t*     tokens;      /* device [rows] */
+    const int32_t*     seq_len;     /* device [1] */
+    uint32_t           rows;
+    uint32_t           max_ctx;     /* >= seq_len[0] + rows */
+    float*             logits;      /* device [vocab], the last row's, or NULL */
+    int32_t*           out_token;   /* device [1]: their argmax, or NULL (needs logits) */
+} opure_prompt_args;
+
+/* workspace of prompt steps of up to `rows` rows */
+int opure_prompt_reserve(opure_dev* dev, const opure_model* model, uint32_t rows, uint32_t max_ctx);
+int opure_prompt_step(opure_dev* dev, const opure_prompt_args* a);
+
 /* ---- one layer of the verify step on a caller's residual: rmsnorm -> fused
  *      QKV GEMV with RoPE and paged K/V append -> paged attention -> o_proj +
  *      residual -> rmsnorm -> gate/up GEMV with SwiGLU -> down + residual, the

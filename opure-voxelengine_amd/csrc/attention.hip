@@ -1191,6 +1191,264 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(CL ? 4
     }
 }
 
+// Attention of a prompt's rows of one sequence (16-bit caches, head_dim 64 or
+// 128): a workgroup takes 64 NT query rows of a KV head (row qi = j group + head,
+// 16 NT a wave; NT 2 once that leaves several workgroups a CU) over tiles of 64 tokens, keeping each row's running maximum, sum
+// and output in registers, so nothing is split, merged or read twice: the
+// split kernel above reads the cache once per 16 positions and writes
+// partials for a combine (1,437 tokens of the 1B shape 230 us a layer, 43
+// here).  Tiles go through LDS in two stages, the next one's loads in flight
+// while a tile computes; the operand mapping, the exponential and the parts of
+// P are k_attn_mfma's.  In LDS the 16-byte pieces of a K row (token) and of a V
+// row (channel) are rotated by an xor key that gives any 8 lanes of a fragment
+// read 8 bank groups.  Bound by the softmax's vector instructions (about 16 a
+// score, 2.5 times the matrix work).  A row's result depends on its position
+// alone: tiles start at multiples of 64 from position 0.
+template <int HD, int AF, int NT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_attn_prompt(AttnParams p)
+{
+    constexpr uint32_t KS = HD / 32u, DT = HD / 16u, TT = 64, WR = 16u * NT, PPR = HD / 8u, NP = TT * PPR / 256u;
+    constexpr uint32_t PG = TT / OPURE_PAGE_SIZE;          // pages a tile
+    constexpr bool P3 = AF == OPURE_A_BF16;
+    __shared__ u4v kt[2][TT * PPR];
+    __shared__ u4v vt[2][HD * TT / 8u];
+    const uint32_t kh = blockIdx.x, q0 = (gridDim.y - 1u - blockIdx.y) * 4u * WR;   // the longest rows first
+    const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63u, g = lane >> 4, r = lane & 15u;
+    const uint32_t group = p.n_heads / p.n_kv, R = p.rows, Gq = group * R;
+    const int32_t* pt = p.page_table;
+    const uint8_t* pool = static_cast<const uint8_t*>(p.pool);
+    const uint32_t nan2 = AF == OPURE_A_F16 ? 0x7E007E00u : 0x7FC07FC0u;
+    const uint32_t ctx = static_cast<uint32_t>(p.seq_len[0]), total = ctx + R;
+    const uint32_t end = ctx + min(q0 + 4u * WR - 1u, Gq - 1u) / group + 1u;             // tokens the workgroup's rows see
+    uint32_t tiles = (end + TT - 1u) / TT;
+    if (tiles > p.nch)
+    {
+        // rows past max_ctx: clamped, reported
+        tiles = p.nch;
+        if (tid == 0u && p.err) p.err[ERR_POSITION] = 1u;
+    }
+    u4v qop[NT][KS];
+    uint32_t lim[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+    {
+        const uint32_t qi = min(q0 + WR * wave + 16u * n + r, Gq - 1u);
+        const uint32_t j = qi / group, head = kh * group + (qi - j * group);
+        lim[n] = ctx + j;
+        const uint8_t* qrow = static_cast<const uint8_t*>(p.q) + ((static_cast<uint64_t>(j) * p.n_heads + head) * HD) * 2u;
+#pragma unroll
+        for (uint32_t s = 0; s < KS; ++s) qop[n][s] = *reinterpret_cast<const u4v*>(qrow + (32u * s + 8u * g) * 2u);
+    }
+    const uint32_t lim_wave = ctx + min(q0 + WR * wave, Gq - 1u) / group;        // the wave's first row's
+    // piece u of this thread: K token kt_, piece kc; V page vp (the same page), channel vd, half vh.  2 HD pieces a page.
+    uint32_t pgi[NP], ktok[NP], kdst[NP], vtok[NP], vdst[NP];
+    uint64_t koff[NP], voff[NP];
+    const uint64_t plane = static_cast<uint64_t>(OPURE_PAGE_SIZE) * HD;
+#pragma unroll
+    for (uint32_t u = 0; u < NP; ++u)
+    {
+        const uint32_t e = u * 256u + tid;
+        pgi[u] = e / (2u * HD);
+        const uint32_t t = e / PPR, c = e % PPR;
+        ktok[u] = t;
+        kdst[u] = t * PPR + (c ^ ((t & 3u) | (((t >> 3) & 1u) << 2)));
+        koff[u] = (static_cast<uint64_t>(t % OPURE_PAGE_SIZE) * HD + 8u * c) * 2u;
+        const uint32_t w = e % (2u * HD), d = w >> 1, h = w & 1u;
+        vtok[u] = pgi[u] * OPURE_PAGE_SIZE + 8u * h;
+        vdst[u] = d * 8u + ((2u * pgi[u] + h) ^ (d & 7u));
+        voff[u] = (static_cast<uint64_t>(d) * OPURE_PAGE_SIZE + 8u * h) * 2u;
+    }
+    auto entries = [&](uint32_t tile, int32_t (&pe)[NP]) {
+#pragma unroll
+        for (uint32_t u = 0; u < NP; ++u) pe[u] = pt[min(tile * PG + pgi[u], p.max_pages - 1u)];
+    };
+    auto valid = [&](uint32_t tile, uint32_t u, int32_t pg) {
+        return tile * PG + pgi[u] < p.max_pages && pg >= 0 && static_cast<uint32_t>(pg) < p.n_pages;
+    };
+    u4v kv_[NP], vv[NP];
+    int32_t pe[NP], cur[NP];
+    auto load = [&](uint32_t tile) {
+#pragma unroll
+        for (uint32_t u = 0; u < NP; ++u)
+        {
+            cur[u] = valid(tile, u, pe[u]) ? pe[u] : -1;
+            const uint64_t pg = cur[u] >= 0 ? static_cast<uint32_t>(cur[u]) : 0u;
+            const uint64_t base = ((static_cast<uint64_t>(p.layer) * p.n_pages + pg) * 2u * p.n_kv + kh) * plane * 2u;
+            kv_[u] = *reinterpret_cast<const u4v*>(pool + base + koff[u]);
+            vv[u] = *reinterpret_cast<const u4v*>(pool + base + p.n_kv * plane * 2u + voff[u]);
+        }
+    };
+    // a missing page reads NaN, slots past the cache 0
+    auto store = [&](uint32_t tile) {
+        u4v* k = kt[tile & 1u];
+        u4v* v = vt[tile & 1u];
+        const bool tail = (tile + 1u) * TT > total;        // uniform
+#pragma unroll
+        for (uint32_t u = 0; u < NP; ++u)
+        {
+            u4v a = cur[u] >= 0 ? kv_[u] : u4v{nan2, nan2, nan2, nan2};
+            u4v b = cur[u] >= 0 ? vv[u] : u4v{nan2, nan2, nan2, nan2};
+            if (tail)
+            {
+                const u4v z = {0u, 0u, 0u, 0u};
+                const uint32_t tk = tile * TT + ktok[u], tv = tile * TT + vtok[u];
+                if (tk >= total) a = z;
+                if (tv >= total) b = z;
+                else if (tv + 8u > total) b = mask_tail<AF>(b, total - tv);
+            }
+            k[kdst[u]] = a;
+            v[vdst[u]] = b;
+        }
+    };
+    f4_t o[DT][NT];
+    float m[NT], l[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+    {
+        m[n] = -__builtin_huge_valf();
+        l[n] = 0.0f;
+#pragma unroll
+        for (uint32_t dt = 0; dt < DT; ++dt) o[dt][n] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    entries(0u, pe);
+    load(0u);
+    entries(1u, pe);
+    for (uint32_t tile = 0; tile < tiles; ++tile)
+    {
+        store(tile);
+        __syncthreads();
+        if (tile + 1u < tiles)
+        {
+            load(tile + 1u);
+            entries(tile + 2u, pe);
+        }
+        const u4v* k = kt[tile & 1u];
+        const u4v* v = vt[tile & 1u];
+        const uint32_t t0 = tile * TT;
+        const bool masked = t0 + TT - 1u > lim_wave;       // uniform over the wave
+        float sc[2][2][NT][4];
+#pragma unroll
+        for (uint32_t kk = 0; kk < 2; ++kk)
+#pragma unroll
+            for (uint32_t T = 0; T < 2; ++T)
+            {
+                const uint32_t tr = 32u * kk + 8u * (r >> 2) + (r & 3u) + 4u * T;
+                const uint32_t key = (tr & 3u) | (((tr >> 3) & 1u) << 2);
+                f4_t acc[NT];
+#pragma unroll
+                for (int n = 0; n < NT; ++n) acc[n] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (uint32_t s = 0; s < KS; ++s)
+                {
+                    const u4v kf = k[tr * PPR + ((4u * s + g) ^ key)];
+#pragma unroll
+                    for (int n = 0; n < NT; ++n) acc[n] = mfma32<AF>(kf, qop[n][s], acc[n]);
+                }
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) sc[kk][T][n][i] = __fmul_rn(acc[n][i], p.scale);
+            }
+        if (masked)
+#pragma unroll
+            for (uint32_t kk = 0; kk < 2; ++kk)
+#pragma unroll
+                for (uint32_t T = 0; T < 2; ++T)
+#pragma unroll
+                    for (int n = 0; n < NT; ++n)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            if (t0 + 32u * kk + 8u * g + 4u * T + i > lim[n]) sc[kk][T][n][i] = -__builtin_huge_valf();
+        u4v pop[2][NT], plo[2][NT], plo2[2][NT];
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+        {
+            float mx = -__builtin_huge_valf();
+#pragma unroll
+            for (uint32_t kk = 0; kk < 2; ++kk)
+#pragma unroll
+                for (uint32_t T = 0; T < 2; ++T)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) mx = fmaxf(mx, sc[kk][T][n][i]);
+            mx = fmaxf(m[n], max_xor32(max_xor16(mx)));
+            // the rows' outputs and sums at the new maximum (left as they are while no row's moves)
+            if (__any(mx != m[n]))
+            {
+                const float a = m[n] == -__builtin_huge_valf() ? 0.0f : exp_hw(__fsub_rn(m[n], mx));
+                l[n] = __fmul_rn(l[n], a);
+#pragma unroll
+                for (uint32_t dt = 0; dt < DT; ++dt)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) o[dt][n][i] = __fmul_rn(o[dt][n][i], a);
+                m[n] = mx;
+            }
+            float sum = 0.0f;
+#pragma unroll
+            for (uint32_t kk = 0; kk < 2; ++kk)
+            {
+                float e[8], lo[8];
+#pragma unroll
+                for (uint32_t T = 0; T < 2; ++T)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                    {
+                        const float s = sc[kk][T][n][i];
+                        e[4 * T + i] = s == -__builtin_huge_valf() ? 0.0f : exp_hw(__fsub_rn(s, mx));
+                        sum += e[4 * T + i];
+                    }
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                {
+                    const uint32_t pr = pack_pair<AF>(e[2 * i], e[2 * i + 1]);
+                    pop[kk][n][i] = pr;
+                    lo[2 * i] = __fsub_rn(e[2 * i], unpack_lo<AF>(pr));
+                    lo[2 * i + 1] = __fsub_rn(e[2 * i + 1], unpack_hi<AF>(pr));
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                {
+                    const uint32_t pr = pack_pair<AF>(lo[2 * i], lo[2 * i + 1]);
+                    plo[kk][n][i] = pr;
+                    if constexpr (P3)
+                        plo2[kk][n][i] = pack_pair<AF>(__fsub_rn(lo[2 * i], unpack_lo<AF>(pr)),
+                                                       __fsub_rn(lo[2 * i + 1], unpack_hi<AF>(pr)));
+                }
+            }
+            l[n] += sum;                                   // this lane group's share
+        }
+#pragma unroll
+        for (uint32_t kk = 0; kk < 2; ++kk)
+#pragma unroll
+            for (uint32_t dt = 0; dt < DT; ++dt)
+            {
+                const uint32_t d = 16u * dt + r;
+                const u4v vf = v[d * 8u + ((4u * kk + g) ^ (d & 7u))];
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+                {
+                    if constexpr (P3) o[dt][n] = mfma32<AF>(vf, plo2[kk][n], o[dt][n]);
+                    o[dt][n] = mfma32<AF>(vf, plo[kk][n], o[dt][n]);
+                    o[dt][n] = mfma32<AF>(vf, pop[kk][n], o[dt][n]);
+                }
+            }
+    }
+    typedef uint32_t u2v __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+    {
+        const float den = add_xor32(add_xor16(l[n])), dd = den > 0.0f ? den : 1.0f;
+        const uint32_t qi = q0 + WR * wave + 16u * n + r;
+        if (qi >= Gq) continue;
+        const uint32_t j = qi / group, head = kh * group + (qi - j * group);
+        uint8_t* row = static_cast<uint8_t*>(p.out) + ((static_cast<uint64_t>(j) * p.n_heads + head) * HD + 4u * g) * 2u;
+#pragma unroll
+        for (uint32_t dt = 0; dt < DT; ++dt)
+            *reinterpret_cast<u2v*>(row + 32u * dt) =
+                u2v{pack_pair<AF>(__fdiv_rn(o[dt][n][0], dd), __fdiv_rn(o[dt][n][1], dd)),
+                    pack_pair<AF>(__fdiv_rn(o[dt][n][2], dd), __fdiv_rn(o[dt][n][3], dd))};
+    }
+}
+
 // One wave per (row, query head): merge that row's items 0..last in order.
 // An item is a partial, or (GRP > 1) a group of GRP chunk partials merged in
 // chunk order by merge_scales/merge_val, as the folded attention kernel merges
@@ -1484,6 +1742,53 @@ int attn_validate(const opure_model* m, const opure_kv* kv, uint32_t batch, uint
         OPURE_REQUIRE(lds <= 160u * 1024u, OPURE_E_CAPACITY, "attention: %u query rows per KV head exceed LDS",
                       group * rows);
     }
+    return OPURE_OK;
+}
+
+int attn_prompt_validate(const opure_model* m, const opure_kv* kv, uint32_t rows, uint32_t max_ctx)
+{
+    OPURE_REQUIRE(rows > OPURE_MAX_ROWS && rows <= OPURE_MAX_PROMPT_ROWS, OPURE_E_CAPACITY,
+                  "prompt attention: %u rows outside %d..%d", rows, OPURE_MAX_ROWS + 1, OPURE_MAX_PROMPT_ROWS);
+    const int rc = attn_validate(m, kv, 1u, 1u, max_ctx);
+    if (rc) return rc;
+    OPURE_REQUIRE(use_mfma(m->afmt) && hd_64_128(m->head_dim), OPURE_E_UNSUPPORTED,
+                  "prompt attention: built for 16-bit caches and head_dim 64 or 128, not %s and %u", afmt_name(m->afmt),
+                  m->head_dim);
+    OPURE_REQUIRE(max_ctx >= rows, OPURE_E_CAPACITY, "prompt attention: max_ctx %u below %u rows", max_ctx, rows);
+    return OPURE_OK;
+}
+
+int attn_prompt_launch(opure_dev* dev, const opure_model* m, const opure_kv* kv, uint32_t layer, uint32_t rows,
+                       const int32_t* seq_len, uint32_t max_ctx, const void* q, void* out)
+{
+    AttnParams p{};
+    p.q = q;
+    p.out = out;
+    p.pool = kv->pool;
+    p.page_table = kv->page_table;
+    p.seq_len = seq_len;
+    p.n_heads = m->n_heads;
+    p.n_kv = m->n_kv_heads;
+    p.hd = m->head_dim;
+    p.rows = rows;
+    p.n_pages = kv->n_pages;
+    p.max_pages = kv->max_pages_per_seq;
+    p.layer = layer;
+    p.nch = (max_ctx + 63u) / 64u;
+    p.scale = m->attn_scale;
+    p.err = dev->err;
+    const uint32_t Gq = rows * (p.n_heads / p.n_kv), n_cu = dev->n_cu > 0 ? static_cast<uint32_t>(dev->n_cu) : 256u;
+    // 128 rows a workgroup read each tile from LDS for twice the work, once
+    // there are four such workgroups a CU to overlap; below, 64
+    const bool two = static_cast<uint64_t>(p.n_kv) * ((Gq + 127u) / 128u) >= 4ull * n_cu;
+    const dim3 grid(p.n_kv, two ? (Gq + 127u) / 128u : (Gq + 63u) / 64u);
+    auto go = [&](auto one, auto pair) { OPURE_LAUNCH(dev, (two ? pair : one), grid, dim3(256), 0, p); };
+    const bool h = m->afmt == OPURE_A_F16;
+    if (p.hd == 64u && h) go(&k_attn_prompt<64, OPURE_A_F16, 1>, &k_attn_prompt<64, OPURE_A_F16, 2>);
+    else if (p.hd == 64u) go(&k_attn_prompt<64, OPURE_A_BF16, 1>, &k_attn_prompt<64, OPURE_A_BF16, 2>);
+    else if (h) go(&k_attn_prompt<128, OPURE_A_F16, 1>, &k_attn_prompt<128, OPURE_A_F16, 2>);
+    else go(&k_attn_prompt<128, OPURE_A_BF16, 1>, &k_attn_prompt<128, OPURE_A_BF16, 2>);
+    OPURE_LAUNCH_CHECK("k_attn_prompt");
     return OPURE_OK;
 }
 

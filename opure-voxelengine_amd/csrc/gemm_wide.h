@@ -53,24 +53,22 @@ constexpr uint32_t WIDE_MAX_M = 256;  // rows of X
 //     stream: no matrix work on column tiles that are not there, and at one
 //     tile a wave twice the workgroups (8B o_proj, 4 splits: 128 -> 256), so
 //     every CU loads: uint4 gate/up 28,672 x 4,096 at 24 rows 77.5 -> 26.3 us.
-template <uint32_t TA_, uint32_t TB_, uint32_t WC_> struct WideShape {
-    static constexpr uint32_t TA = TA_, TB = TB_, WC = WC_, RT = (4u / WC_) * TA_, CT = WC_ * TB_;
+// KH = 2 runs two sets of 4 waves on alternate K blocks (two waves a SIMD: one
+// issues MFMAs while the other waits); the uint4 kernel's registers leave room
+// for one.
+template <uint32_t TA_, uint32_t TB_, uint32_t WC_, uint32_t KH_> struct WideShape {
+    static constexpr uint32_t TA = TA_, TB = TB_, WC = WC_, KH = KH_, RT = (4u / WC_) * TA_, CT = WC_ * TB_, NTH = 256u * KH_;
 };
 
 // register slots of the software pipeline: DW weight blocks and DX X blocks
 // in flight; the K loop is unrolled by U = lcm(DW, DX), an even number, so
-// slots and LDS stages are compile-time.  KH = 2 runs two sets of 4 waves on
-// alternate K blocks (two waves a SIMD: one issues MFMAs while the other
-// waits); the uint4 kernel's registers leave room for one.  PU: the plan's
-// splits are multiples of PU blocks.
-template <int WF, uint32_t CT> struct WideDepth;
-template <uint32_t CT> struct WideDepth<OPURE_W_I8PC, CT>   { static constexpr uint32_t DW = 4, DX = 2, U = 4, KH = 2, PU = 4; };
-template <uint32_t CT> struct WideDepth<OPURE_W_I4G128, CT>
-{
-    static constexpr uint32_t DW = CT == 8u ? 2 : 4, DX = CT == 8u ? 1 : 2, U = CT == 8u ? 2 : 4, KH = 1, PU = 2;
+// slots and LDS stages are compile-time.
+template <int WF, class SH> struct WideDepth {
+    static constexpr bool FEW = SH::CT < 8u, I8 = WF == OPURE_W_I8PC;
+    static constexpr uint32_t DW = I8 ? (SH::KH == 2u ? 4 : 2) : (FEW && SH::TA == 1u ? 4 : 2), DX = I8 ? 2 : (FEW ? 2 : 1), U = DW > DX ? DW : DX;
 };
-
-constexpr uint32_t wide_threads(int wf) { return wf == OPURE_W_I8PC ? 512u : 256u; }   // 256 KH
+// the plan's splits are multiples of this many blocks
+constexpr uint32_t wide_split_unit(uint32_t wf) { return wf == OPURE_W_I8PC ? 4u : 2u; }
 
 struct WParams {
     KParams p;        // shape, pointers, epilogue
@@ -82,6 +80,7 @@ struct WParams {
     uint32_t bps;     // blocks per split
     uint32_t part_rows;  // splits > 1: 0 = accumulators [split][tile][mt][64] lanes, 1 = [split][M][out] rows
     f4_t* part;       // splits > 1: the splits' accumulators
+    uint32_t prompt;  // host: more rows than a batch (a prompt's step)
 };
 
 // Workgroup -> (split, row group, column group).  Workgroups are dispatched
@@ -100,7 +99,7 @@ __device__ __forceinline__ void wide_coords(const WParams& wp, uint32_t& split, 
 }
 
 template <int WF, int AF, int EPI, class SH>
-__global__ __launch_bounds__(wide_threads(WF)) __attribute__((amdgpu_waves_per_eu(2))) void k_gemm_wide(WParams wp)
+__global__ __launch_bounds__(SH::NTH) __attribute__((amdgpu_waves_per_eu(2))) void k_gemm_wide(WParams wp)
 {
     static_assert(WF == OPURE_W_I8PC || WF == OPURE_W_I4G128, "the wide GEMV reads quantised weights");
     constexpr uint32_t KB = Fmt<WF>::KB;
@@ -109,8 +108,9 @@ __global__ __launch_bounds__(wide_threads(WF)) __attribute__((amdgpu_waves_per_e
     constexpr uint32_t TA = SH::TA, TB = SH::TB, WC = SH::WC, RT = SH::RT, CT = SH::CT;
     constexpr uint32_t XR = CT * 16u * CH / 256u;  // X chunks a thread stages per block
     constexpr uint32_t STAGE = CT * NMF * 64u;     // u4_t per LDS stage
-    using WD = WideDepth<WF, CT>;
-    constexpr uint32_t DW = WD::DW, DX = WD::DX, U = WD::U, KH = WD::KH;
+    using WD = WideDepth<WF, SH>;
+    constexpr uint32_t DW = WD::DW, DX = WD::DX, U = WD::U, KH = SH::KH;
+    static_assert(U % 2 == 0 && U % DX == 0 && U % DW == 0, "static slots and stages");
     constexpr bool GS = WF == OPURE_W_I4G128;      // group sums of X
     static_assert(XR >= 1 && TB % 2 == 0, "whole chunks a thread; the halves exchange half of the column tiles");
     static_assert(KH == 1 || 4u * TA * TB * 64u <= KH * 2u * STAGE, "the halves' exchange reuses the X stages");
@@ -505,8 +505,6 @@ int launch_wide_reduce_norm(opure_dev* dev, const WParams& wp, const float* gain
     return OPURE_OK;
 }
 
-using WIDE_BIG = WideShape<2, 8, 1>;
-
 template <int WF, int AF, int EPI>
 int launch_wide_epi_only(opure_dev* dev, const WParams& wp)
 {
@@ -517,13 +515,19 @@ int launch_wide_epi_only(opure_dev* dev, const WParams& wp)
         WParams q = wp;
         q.nrg = (wp.p.tiles + SH::RT - 1u) / SH::RT;
         OPURE_LAUNCH(dev, (k_gemm_wide<WF, AF, EPI, SH>), dim3(q.nrg * q.ncg * q.splits),
-                     dim3(wide_threads(WF)), 0, q);
+                     dim3(SH::NTH), 0, q);
         OPURE_LAUNCH_CHECK("k_gemm_wide");
         return OPURE_OK;
     };
-    if (wp.cgs <= 2u) return go(WideShape<1, 2, 1>{});
-    if (wp.cgs <= 4u) return go(WideShape<1, 4, 1>{});
-    return go(WIDE_BIG{});
+    constexpr uint32_t KH = WF == OPURE_W_I8PC ? 2u : 1u;
+    // a prompt's step has workgroups enough for two and more a CU: one set of
+    // waves a workgroup, each wave four weight tiles
+    if (wp.prompt && wp.cgs <= 4u) return go(WideShape<4, 2, 2, 1>{});
+    if constexpr (WF == OPURE_W_I8PC)
+        if (wp.prompt) return go(WideShape<4, 4, 2, 1>{});
+    if (wp.cgs <= 2u) return go(WideShape<1, 2, 1, KH>{});
+    if (wp.cgs <= 4u) return go(WideShape<1, 4, 1, KH>{});
+    return go(WideShape<2, 8, 1, KH>{});
 }
 
 template <int WF, int AF, int EPI>

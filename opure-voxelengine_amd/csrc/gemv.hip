@@ -251,18 +251,28 @@ WidePlan wide_plan(const opure_dev* dev, uint32_t wfmt, uint32_t out, uint32_t i
     using namespace opure_gemv;
     WidePlan w;
     const uint32_t KB = kb_of(wfmt);
-    const uint32_t U = wfmt == OPURE_W_I8PC ? WideDepth<OPURE_W_I8PC, WIDE_CG>::PU : WideDepth<OPURE_W_I4G128, WIDE_CG>::PU;
+    const uint32_t U = wide_split_unit(wfmt);
     w.tiles = out / 16u;
     w.nblk = in / KB;
     w.mt = (M + 15u) / 16u;
     w.nrg = (w.tiles + WIDE_RT - 1u) / WIDE_RT;
+    const uint32_t cus = dev && dev->n_cu > 0 ? static_cast<uint32_t>(dev->n_cu) : 256u;
     w.ncg = (w.mt + WIDE_CG - 1u) / WIDE_CG;
+    // a prompt's step with one to two workgroups a CU: column groups of half
+    // the size (1B qkv over 1,436 rows: 288 workgroups -> 552, 54 -> 47 us).
+    // Fewer workgroups are split over K instead (o_proj and down, 192: 36 and
+    // 87 us with the next rmsnorm, 37 and 109 in halves).
+    const uint32_t wgs = w.nrg * w.ncg;
+    if (M > OPURE_MAX_BATCH_ROWS && wgs >= cus && wgs < 2u * cus) w.ncg = (w.mt + WIDE_CG / 2u - 1u) / (WIDE_CG / 2u);
     w.cgs = (w.mt + w.ncg - 1u) / w.ncg;
     // split K while there are fewer row groups than half the CUs (a batch
     // over 128 rows has two column groups), at most 8 ways and U blocks a split
-    const uint32_t n_cu = dev && dev->n_cu > 0 ? static_cast<uint32_t>(dev->n_cu) : 256u;
-    const uint32_t want = std::max(1u, n_cu / 2u);
+    const uint32_t want = std::max(1u, cus / 2u);
     if (w.nrg < want) w.splits = std::min({(want + w.nrg - 1u) / w.nrg, std::max(1u, w.nblk / U), 8u});
+    // a prompt's step: its column groups fill the chip without splits (whose
+    // accumulators would be written and read back), unless there are few
+    if (M > OPURE_MAX_BATCH_ROWS)
+        w.splits = std::min({(cus + w.nrg * w.ncg - 1u) / (w.nrg * w.ncg), std::max(1u, w.nblk / U), 8u});
     w.bps = (w.nblk + w.splits - 1u) / w.splits;
     w.bps = (w.bps + U - 1u) / U * U;
     w.splits = (w.nblk + w.bps - 1u) / w.bps;
@@ -305,8 +315,8 @@ int gemv_validate(const GemvCall& c)
     const uint32_t want = c.epi == EPI_SWIGLU ? OPURE_LAYOUT_TILED_SWIGLU : OPURE_LAYOUT_TILED;
     OPURE_REQUIRE(c.W.layout == want, OPURE_E_INVALID,
                   "gemv: weights must be in layout %u (opure_tile_linear), got %u", want, c.W.layout);
-    OPURE_REQUIRE(c.M >= 1 && c.M <= OPURE_MAX_BATCH_ROWS, OPURE_E_CAPACITY, "gemv: M=%u outside 1..%d", c.M,
-                  OPURE_MAX_BATCH_ROWS);
+    const uint32_t most = c.prompt ? OPURE_MAX_PROMPT_ROWS : OPURE_MAX_BATCH_ROWS;
+    OPURE_REQUIRE(c.M >= 1 && c.M <= most, OPURE_E_CAPACITY, "gemv: M=%u outside 1..%u", c.M, most);
     if (c.M > OPURE_MAX_ROWS)
     {
         OPURE_REQUIRE(wf != OPURE_W_F32 && af != OPURE_A_F32, OPURE_E_UNSUPPORTED,
@@ -385,6 +395,7 @@ static int gemv_launch_wide(opure_dev* dev, const GemvCall& c)
     wp.splits = w.splits;
     wp.bps = w.bps;
     wp.part = static_cast<f4_t*>(c.part_scratch);
+    wp.prompt = c.M > OPURE_MAX_BATCH_ROWS ? 1u : 0u;
     kp.eps = c.eps;
     // a residual with K splits and the next rmsnorm: row-major partials, added
     // and normalised per row by k_wide_reduce_norm (outputs up to 4096)

@@ -227,6 +227,8 @@ struct GemvCall {
     // to norm_out [M][out] in xfmt (the same bits as the consumer's own pass)
     const float* norm_gain = nullptr;
     void* norm_out = nullptr;
+    // a prompt's step: up to OPURE_MAX_PROMPT_ROWS rows
+    bool prompt = false;
     QkvEpilogue qkv{};
     LogitsEpilogue logits{};
 };
@@ -248,6 +250,10 @@ uint32_t tiled_block_k(uint32_t wfmt);      // k values per 64-byte block
 uint64_t attn_partial_bytes(uint32_t batch, uint32_t n_kv, uint32_t group, uint32_t rows, uint32_t hd, uint32_t afmt,
                             uint32_t max_ctx);
 int      attn_validate(const opure_model* m, const opure_kv* kv, uint32_t batch, uint32_t rows, uint32_t max_ctx);
+// a prompt's rows of one sequence (16-bit caches, head_dim 64 or 128)
+int      attn_prompt_validate(const opure_model* m, const opure_kv* kv, uint32_t rows, uint32_t max_ctx);
+int      attn_prompt_launch(opure_dev* dev, const opure_model* m, const opure_kv* kv, uint32_t layer, uint32_t rows,
+                            const int32_t* seq_len, uint32_t max_ctx, const void* q, void* out);
 int      attn_launch(opure_dev* dev, const opure_model* m, const opure_kv* kv, uint32_t layer, uint32_t batch,
                      uint32_t rows, const int32_t* seq_len, uint32_t max_ctx, const void* q, void* out, float* part);
 

@@ -122,16 +122,26 @@ __global__ __launch_bounds__(256) void k_tile_sumsq(const float* x, uint32_t M, 
     ss[static_cast<uint64_t>(c16) * M + r] = sq;
 }
 
+// the position of a prompt's last row
+__global__ void k_last_position(const int32_t* seq_len, uint32_t rows, int32_t* out)
+{
+    out[0] = seq_len[0] + static_cast<int32_t>(rows) - 1;
+}
+
 }  // namespace
 
 namespace opure_hip {
 
 struct VerifyPlan {
+    uint64_t last = 0, ss1 = 0;   // prompt: the last row's position and sums of squares
     uint64_t x = 0, ss = 0, xn = 0, q = 0, att = 0, h = 0, am_val = 0, am_idx = 0, attn = 0, rej = 0, part = 0, total = 0;
     uint32_t lm_tiles = 0;
 };
 
-static VerifyPlan make_plan(const opure_dev* dev, const opure_model* m, uint32_t B, uint32_t R, uint32_t max_ctx)
+// prompt: one sequence's R rows, of which only the last gets (split) attention
+// in the last layer, logits and their argmax
+static VerifyPlan make_plan(const opure_dev* dev, const opure_model* m, uint32_t B, uint32_t R, uint32_t max_ctx,
+                            bool prompt = false)
 {
     VerifyPlan p;
     const uint64_t MR = static_cast<uint64_t>(B) * R;
@@ -148,17 +158,19 @@ static VerifyPlan make_plan(const opure_dev* dev, const opure_model* m, uint32_t
     // argmax partials: one per LM-head workgroup and row (at most one per tile),
     // or one per 4096 logits when more than OPURE_MAX_ROWS rows store the logits
     p.lm_tiles = m->vocab / 16u;
-    const uint64_t am = std::max<uint64_t>(p.lm_tiles, argmax_parts(m->vocab)) * MR * 4u;
+    const uint64_t am = std::max<uint64_t>(p.lm_tiles, argmax_parts(m->vocab)) * (prompt ? 1u : MR) * 4u;
     p.am_val = take(am);
     p.am_idx = take(am);
-    p.attn = take(attn_partial_bytes(B, m->n_kv_heads, m->n_heads / m->n_kv_heads, R, m->head_dim, m->afmt, max_ctx));
-    p.rej = take(accept_ws_bytes(B, R - 1u, m->vocab, OPURE_ACCEPT_REJECTION));
+    p.attn = take(attn_partial_bytes(B, m->n_kv_heads, m->n_heads / m->n_kv_heads, prompt ? 1u : R, m->head_dim, m->afmt, max_ctx));
+    p.rej = take(prompt ? 0u : accept_ws_bytes(B, R - 1u, m->vocab, OPURE_ACCEPT_REJECTION));
     // split-K accumulators of the GEMVs over more than OPURE_MAX_ROWS rows
     uint64_t part = 0;
     for (const auto& s : {std::pair<uint32_t, uint32_t>{qdim + 2u * kvdim, m->hidden}, {m->hidden, qdim},
-                          {2u * m->ffn, m->hidden}, {m->hidden, m->ffn}, {m->vocab, m->hidden}})
-        part = std::max(part, gemv_scratch_bytes(dev, m->wfmt, s.first, s.second, static_cast<uint32_t>(MR)));
+                          {2u * m->ffn, m->hidden}, {m->hidden, m->ffn}, {prompt ? 0u : m->vocab, m->hidden}})
+        if (s.first) part = std::max(part, gemv_scratch_bytes(dev, m->wfmt, s.first, s.second, static_cast<uint32_t>(MR)));
     p.part = take(part);
+    p.last = take(prompt ? 4u : 0u);
+    p.ss1 = take(prompt ? (m->hidden / 16u) * 4u : 0u);
     p.total = off;
     return p;
 }
@@ -174,7 +186,8 @@ static int check_linear(const opure_linear& L, uint32_t out, uint32_t in, const 
     return OPURE_OK;
 }
 
-static int check_model(const opure_model* m, const opure_kv* kv, uint32_t B, uint32_t R, uint32_t max_ctx)
+static int check_model(const opure_model* m, const opure_kv* kv, uint32_t B, uint32_t R, uint32_t max_ctx,
+                       bool prompt = false)
 {
     OPURE_REQUIRE(m && kv && m->layers && m->final_norm && m->rope_cos && m->rope_sin, OPURE_E_INVALID,
                   "verify: null model field");
@@ -186,11 +199,11 @@ static int check_model(const opure_model* m, const opure_kv* kv, uint32_t B, uin
                     (m->wfmt == OPURE_W_I4G128 && (m->afmt == OPURE_A_F16 || m->afmt == OPURE_A_BF16));
     OPURE_REQUIRE(ok, OPURE_E_UNSUPPORTED, "verify: weights %u with %s activations are not built", m->wfmt,
                   afmt_name(m->afmt));
-    int rc = attn_validate(m, kv, B, R, max_ctx);
+    int rc = prompt ? attn_prompt_validate(m, kv, R, max_ctx) : attn_validate(m, kv, B, R, max_ctx);
     if (rc) return rc;
     OPURE_REQUIRE(max_ctx <= m->rope_max_pos, OPURE_E_CAPACITY, "verify: max_ctx %u beyond the RoPE table (%u)", max_ctx,
                   m->rope_max_pos);
-    OPURE_REQUIRE(R >= 1 && R - 1u < 64u, OPURE_E_CAPACITY, "verify: rows %u", R);
+    OPURE_REQUIRE(prompt || (R >= 1 && R - 1u < 64u), OPURE_E_CAPACITY, "verify: rows %u", R);
     const uint32_t qdim = m->n_heads * m->head_dim, kvdim = m->n_kv_heads * m->head_dim;
     if ((rc = check_linear(m->embed, m->vocab, m->hidden, "embed", m->wfmt))) return rc;
     if ((rc = check_linear(m->lm_head, m->vocab, m->hidden, "lm_head", m->wfmt))) return rc;
@@ -207,25 +220,13 @@ static int check_model(const opure_model* m, const opure_kv* kv, uint32_t B, uin
     return OPURE_OK;
 }
 
-// One layer of the verify step on the residual x (fp32 [B*R][hidden]) whose
-// per-tile sums of squares are in ss: rmsnorm + qkv GEMV + RoPE + paged K/V
-// append, attention, o_proj + residual, rmsnorm + gate/up + SwiGLU, down +
-// residual.  `c` carries the step-wide GEMV fields (formats, rows, scratch).
-// The body of RecordForward's layer loop (Opure_VoxelEngine.cpp:296-492).
-// Above OPURE_MAX_ROWS rows a residual GEMV also writes the next rmsnorm's
-// rows (GemvCall::norm_gain) into xn, so the consumer reads them instead of
-// running its own normalisation pass: xn_ready says the incoming xn holds
-// this layer's attention-norm rows, next_gain is the norm after the layer.
-static int layer_launch(opure_dev* dev, const opure_model* m, const opure_kv* kv, uint32_t L, uint32_t B, uint32_t R,
-                        const int32_t* seq_len, uint32_t max_ctx, const VerifyPlan& P, float* x, float* ss, GemvCall& c,
-                        bool xn_ready = false, const float* next_gain = nullptr)
+// rmsnorm + QKV GEMV with RoPE, q stored, K/V appended
+static int qkv_launch(opure_dev* dev, const opure_model* m, const opure_kv* kv, uint32_t L, uint32_t R, const int32_t* seq_len,
+                      const VerifyPlan& P, float* x, float* ss, GemvCall& c, bool xn_ready)
 {
-    const bool wide = B * R > OPURE_MAX_ROWS;
     char* ws = static_cast<char*>(dev->ws);
     void* xn = ws + P.xn;
     void* q = ws + P.q;
-    void* att = ws + P.att;
-    void* hbuf = ws + P.h;
     const uint32_t qdim = m->n_heads * m->head_dim, kvdim = m->n_kv_heads * m->head_dim;
     int rc;
     const opure_layer_weights& W = m->layers[L];
@@ -256,12 +257,20 @@ static int layer_launch(opure_dev* dev, const opure_model* m, const opure_kv* kv
     if ((rc = gemv_validate(c)) || (rc = prof_begin(dev, OPURE_STAGE_QKV)) || (rc = gemv_launch(dev, c)) ||
         (rc = prof_end(dev)))
         return rc;
+    return OPURE_OK;
+}
 
-    if ((rc = prof_begin(dev, OPURE_STAGE_ATTN)) ||
-        (rc = attn_launch(dev, m, kv, L, B, R, seq_len, max_ctx, q, att, reinterpret_cast<float*>(ws + P.attn))) ||
-        (rc = prof_end(dev)))
-        return rc;
-
+// o_proj + residual, rmsnorm + gate/up + SwiGLU, down + residual over c.M rows
+static int post_attention_launch(opure_dev* dev, const opure_model* m, uint32_t L, const VerifyPlan& P, float* x, float* ss,
+                                 GemvCall& c, const float* next_gain)
+{
+    const bool wide = c.M > OPURE_MAX_ROWS;
+    char* ws = static_cast<char*>(dev->ws);
+    void* xn = ws + P.xn;
+    void* att = ws + P.att;
+    void* hbuf = ws + P.h;
+    int rc;
+    const opure_layer_weights& W = m->layers[L];
     c.W = W.o;
     c.x = att;
     c.gain = nullptr;
@@ -302,6 +311,32 @@ static int layer_launch(opure_dev* dev, const opure_model* m, const opure_kv* kv
     return OPURE_OK;
 }
 
+// One layer of the verify step on the residual x (fp32 [B*R][hidden]) whose
+// per-tile sums of squares are in ss: rmsnorm + qkv GEMV + RoPE + paged K/V
+// append, attention, o_proj + residual, rmsnorm + gate/up + SwiGLU, down +
+// residual.  `c` carries the step-wide GEMV fields (formats, rows, scratch).
+// The body of RecordForward's layer loop (Opure_VoxelEngine.cpp:296-492).
+// Above OPURE_MAX_ROWS rows a residual GEMV also writes the next rmsnorm's
+// rows (GemvCall::norm_gain) into xn, so the consumer reads them instead of
+// running its own normalisation pass: xn_ready says the incoming xn holds
+// this layer's attention-norm rows, next_gain is the norm after the layer.
+static int layer_launch(opure_dev* dev, const opure_model* m, const opure_kv* kv, uint32_t L, uint32_t B, uint32_t R,
+                        const int32_t* seq_len, uint32_t max_ctx, const VerifyPlan& P, float* x, float* ss, GemvCall& c,
+                        bool xn_ready = false, const float* next_gain = nullptr)
+{
+    char* ws = static_cast<char*>(dev->ws);
+    void* q = ws + P.q;
+    void* att = ws + P.att;
+    int rc;
+    if ((rc = qkv_launch(dev, m, kv, L, R, seq_len, P, x, ss, c, xn_ready))) return rc;
+    if ((rc = prof_begin(dev, OPURE_STAGE_ATTN)) ||
+        (rc = c.prompt ? attn_prompt_launch(dev, m, kv, L, R, seq_len, max_ctx, q, att)
+                       : attn_launch(dev, m, kv, L, B, R, seq_len, max_ctx, q, att, reinterpret_cast<float*>(ws + P.attn))) ||
+        (rc = prof_end(dev)))
+        return rc;
+    return post_attention_launch(dev, m, L, P, x, ss, c, next_gain);
+}
+
 // The GEMV fields shared by every launch of a step over B*R rows.
 static GemvCall step_gemv(const opure_model* m, uint32_t MR, const VerifyPlan& P, char* ws, float* ss)
 {
@@ -331,6 +366,78 @@ int opure_verify_reserve(opure_dev* dev, const opure_model* model, uint32_t batc
                   OPURE_MAX_ROWS, OPURE_MAX_BATCH_ROWS);
     const VerifyPlan p = make_plan(dev, model, batch, rows, max_ctx);
     return ensure_workspace(dev, p.total);
+}
+
+int opure_prompt_reserve(opure_dev* dev, const opure_model* model, uint32_t rows, uint32_t max_ctx)
+{
+    OPURE_REQUIRE(dev && model, OPURE_E_INVALID, "opure_prompt_reserve: null argument");
+    OPURE_REQUIRE(rows > OPURE_MAX_ROWS && rows <= OPURE_MAX_PROMPT_ROWS, OPURE_E_CAPACITY,
+                  "opure_prompt_reserve: %u rows outside %d..%d", rows, OPURE_MAX_ROWS + 1, OPURE_MAX_PROMPT_ROWS);
+    // the K splits, and with them the scratch, follow from the row count: up to
+    // a batch's rows by the weight shape, past that by the column groups
+    uint64_t need = 0;
+    for (uint32_t r = OPURE_MAX_ROWS + 1u; r <= rows; ++r) need = std::max(need, make_plan(dev, model, 1u, r, max_ctx, true).total);
+    return ensure_workspace(dev, need);
+}
+
+int opure_prompt_step(opure_dev* dev, const opure_prompt_args* a)
+{
+    OPURE_REQUIRE(dev && a && a->model && a->kv && a->tokens && a->seq_len && (a->logits || !a->out_token), OPURE_E_INVALID,
+                  "opure_prompt_step: null argument");
+    const opure_model* m = a->model;
+    const uint32_t R = a->rows;
+    int rc = check_model(m, a->kv, 1u, R, a->max_ctx, true);
+    if (rc) return rc;
+    const VerifyPlan P = make_plan(dev, m, 1u, R, a->max_ctx, true);
+    if ((rc = ensure_workspace(dev, P.total))) return rc;
+    char* ws = static_cast<char*>(dev->ws);
+    float* x = reinterpret_cast<float*>(ws + P.x);
+    float* ss = reinterpret_cast<float*>(ws + P.ss);
+    if ((rc = prof_begin(dev, OPURE_STAGE_EMBED))) return rc;
+    OPURE_LAUNCH(dev, k_embed, dim3(R), dim3(256), 0, a->tokens, m->embed, m->wfmt, m->hidden, m->vocab, R,
+                 tiled_block_k(m->wfmt), x, ss, dev->err);
+    OPURE_LAUNCH_CHECK("k_embed");
+    if ((rc = prof_end(dev))) return rc;
+    GemvCall c = step_gemv(m, R, P, ws, ss);
+    c.prompt = true;
+    const uint32_t last = m->n_layers - 1u;
+    for (uint32_t L = 0; L < last; ++L)
+        if ((rc = layer_launch(dev, m, a->kv, L, 1u, R, a->seq_len, a->max_ctx, P, x, ss, c, L > 0u, m->layers[L + 1u].attn_norm)))
+            return rc;
+    // the last layer: every row's K and V, and the rest for the row whose
+    // logits are wanted -- nothing reads the others' outputs
+    if ((rc = qkv_launch(dev, m, a->kv, last, R, a->seq_len, P, x, ss, c, last > 0u)) || !a->logits) return rc;
+    int32_t* pos = reinterpret_cast<int32_t*>(ws + P.last);
+    float* x1 = x + static_cast<uint64_t>(R - 1u) * m->hidden;
+    float* ss1 = reinterpret_cast<float*>(ws + P.ss1);
+    if ((rc = prof_begin(dev, OPURE_STAGE_ATTN))) return rc;
+    OPURE_LAUNCH(dev, k_last_position, dim3(1), dim3(1), 0, a->seq_len, R, pos);
+    OPURE_LAUNCH_CHECK("k_last_position");
+    const uint64_t qrow = static_cast<uint64_t>(R - 1u) * m->n_heads * m->head_dim * act_bytes(m->afmt);
+    if ((rc = attn_launch(dev, m, a->kv, last, 1u, 1u, pos, a->max_ctx, ws + P.q + qrow, ws + P.att,
+                          reinterpret_cast<float*>(ws + P.attn))) ||
+        (rc = prof_end(dev)))
+        return rc;
+    GemvCall c1 = step_gemv(m, 1u, P, ws, ss1);
+    if ((rc = post_attention_launch(dev, m, last, P, x1, ss1, c1, nullptr))) return rc;
+    c1.W = m->lm_head;
+    c1.x = x1;
+    c1.gain = m->final_norm;
+    c1.ss_out = nullptr;
+    c1.y = a->logits;
+    c1.yfmt = OPURE_A_F32;
+    c1.epi = EPI_LOGITS;
+    c1.logits.am_val = reinterpret_cast<float*>(ws + P.am_val);
+    c1.logits.am_idx = reinterpret_cast<int32_t*>(ws + P.am_idx);
+    if ((rc = gemv_validate(c1)) || (rc = prof_begin(dev, OPURE_STAGE_LM_HEAD)) || (rc = gemv_launch(dev, c1)) ||
+        (rc = prof_end(dev)) || !a->out_token)
+        return rc;
+    // the accepted count of no drafts goes to the position's word
+    if ((rc = prof_begin(dev, OPURE_STAGE_ACCEPT)) ||
+        (rc = greedy_from_partials(dev, c1.logits.am_val, c1.logits.am_idx, gemv_grid(dev, c1), 1u, 0u, pos, 0u, a->out_token, pos,
+                                   nullptr)))
+        return rc;
+    return prof_end(dev);
 }
 
 int opure_debug_workspace(opure_dev* dev, void** ptr, uint64_t* bytes)

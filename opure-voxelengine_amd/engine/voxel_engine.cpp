@@ -42,8 +42,10 @@ void* alloc(opure_dev* dev, uint64_t bytes, const char* what)
 }  // namespace
 
 // Device state of one model: its paged KV pool with the free list of its
-// pages, the sequence's page-table row (host mirror and device copy), the
-// same row 16 times for the 256-row prefill, and the prefill steps.
+// pages, the sequence's page-table row (host mirror and device copy), and the
+// prefill steps.  A quantised model's prompt goes through opure_prompt_step,
+// kPromptRows tokens a step; one whose head size that step is not built for
+// takes 256 rows a verify step (16 parts of 16 rows on 16 copies of the row).
 struct VoxelEngine::ModelState {
     explicit ModelState(uint32_t nPages) : pool(nPages) {}
     opure_model desc{};
@@ -52,7 +54,10 @@ struct VoxelEngine::ModelState {
     PagePool pool;
     std::vector<int32_t> row;       // host mirror of kv.page_table
     bool rowsDirty16 = true;        // kv16's rows lag the row
-    bool wide = false;              // quantised weights and 16-bit activations: 256-row prefill
+    bool prompt = false;            // quantised weights, 16-bit activations, head_dim 64 or 128: prompt steps
+    bool wide = false;              // quantised weights, another head size: 256-row prefill
+    uint32_t promptRows = 0;        // tokens a prompt step
+    int32_t* promptIn = nullptr;    // [promptRows] tokens, then the start position
     std::unique_ptr<Step> prefill;      // 16 rows
     std::unique_ptr<Step> prefillWide;  // 16 parts x 16 rows
 };
@@ -73,6 +78,7 @@ struct VoxelEngine::Step {
 namespace {
 constexpr uint32_t kFreedStride = 2;   // pages one rollback of <= 15 drafts can release: ceil(15 / 16) = 1
 constexpr uint32_t kWideParts = 16;    // 16 parts x 16 rows = 256 prefill rows a launch
+constexpr uint32_t kPromptRows = OPURE_MAX_PROMPT_ROWS;
 }  // namespace
 
 VoxelEngine::VoxelEngine() = default;
@@ -118,7 +124,8 @@ void VoxelEngine::Shutdown()
         free_step(m->prefillWide, true);
         opure_buf_free(dev_, m->kv.pool);
         opure_buf_free(dev_, m->kv.page_table);
-        opure_buf_free(dev_, m->kv16.page_table);
+        if (m->kv16.page_table) opure_buf_free(dev_, m->kv16.page_table);
+        if (m->promptIn) opure_buf_free(dev_, m->promptIn);
     }
     target_.reset();
     draft_.reset();
@@ -170,7 +177,9 @@ void VoxelEngine::Initialize(opure_dev* dev, const opure_model& target, const op
             throw Error(OPURE_E_INVALID, "VoxelEngine::Initialize: model RoPE table shorter than maxPositions");
         auto m = std::make_unique<ModelState>(n_pages);
         m->desc = d;
-        m->wide = d.wfmt != OPURE_W_F32 && d.afmt != OPURE_A_F32;
+        const bool quant = d.wfmt != OPURE_W_F32 && d.afmt != OPURE_A_F32;
+        m->prompt = quant && (d.head_dim == 64u || d.head_dim == 128u) && P > OPURE_MAX_ROWS;
+        m->wide = quant && !m->prompt;
         const uint64_t pool = static_cast<uint64_t>(d.n_layers) * n_pages * 2u * d.n_kv_heads * OPURE_PAGE_SIZE *
                               d.head_dim * act_bytes(d.afmt);
         m->kv.pool = alloc(dev, pool, "kv pool");
@@ -180,8 +189,11 @@ void VoxelEngine::Initialize(opure_dev* dev, const opure_model& target, const op
         m->kv.page_table = static_cast<int32_t*>(alloc(dev, n_pages * 4ull, "page table"));
         m->row.assign(n_pages, -1);
         Check(opure_buf_upload(dev, m->kv.page_table, 0, m->row.data(), n_pages * 4ull), "page table upload");
-        m->kv16 = m->kv;
-        m->kv16.page_table = static_cast<int32_t*>(alloc(dev, kWideParts * n_pages * 4ull, "page table x16"));
+        if (m->wide)
+        {
+            m->kv16 = m->kv;
+            m->kv16.page_table = static_cast<int32_t*>(alloc(dev, kWideParts * n_pages * 4ull, "page table x16"));
+        }
         return m;
     };
     target_ = make_model(target);
@@ -241,6 +253,12 @@ void VoxelEngine::Initialize(opure_dev* dev, const opure_model& target, const op
         if (!m) continue;
         m->prefill = make_step(m, OPURE_MAX_ROWS, nullptr, nullptr, false, false, 1, false);
         Check(opure_verify_reserve(dev, &m->desc, 1, OPURE_MAX_ROWS, P), "verify reserve");
+        if (m->prompt)
+        {
+            m->promptRows = std::min(kPromptRows, P);
+            m->promptIn = static_cast<int32_t*>(alloc(dev, (m->promptRows + 1ull) * 4, "prompt inputs"));
+            Check(opure_prompt_reserve(dev, &m->desc, m->promptRows, P), "prompt reserve");
+        }
         if (m->wide)
         {
             m->prefillWide = make_step(m, OPURE_MAX_ROWS, nullptr, nullptr, false, false, kWideParts, false);
@@ -311,8 +329,43 @@ uint32_t VoxelEngine::Prefill(bool draft, const std::vector<uint32_t>& tokens, u
     if (start + tokens.size() > opts_.maxPositions)
         throw Error(OPURE_E_CAPACITY, "VoxelEngine::Prefill: prompt exceeds maxPositions");
     EnsurePages(*m, start + static_cast<uint32_t>(tokens.size()));
-    const size_t body = wantNext ? tokens.size() - 1 : tokens.size();
+    size_t body = wantNext ? tokens.size() - 1 : tokens.size();
     size_t c = 0;
+    if (m->prompt && tokens.size() > OPURE_MAX_ROWS)
+    {
+        // the last step (17 tokens at least) leaves the next token and its
+        // logits where a decode step would
+        std::vector<int32_t> io(m->promptRows + 1u);
+        const size_t n = tokens.size();
+        while (n - c > OPURE_MAX_ROWS)
+        {
+            size_t left = n - c;
+            if (left > m->promptRows) left = std::min<size_t>(m->promptRows, left - (OPURE_MAX_ROWS + 1u));
+            const uint32_t r = static_cast<uint32_t>(left);
+            const bool last = wantNext && !draft && c + r == n;
+            for (uint32_t i = 0; i < r; ++i) io[i] = static_cast<int32_t>(tokens[c + i]);
+            io[r] = static_cast<int32_t>(start + c);
+            Check(opure_buf_upload(dev_, m->promptIn, 0, io.data(), (r + 1ull) * 4), "prompt upload");
+            opure_prompt_args a{};
+            a.model = &m->desc;
+            a.kv = &m->kv;
+            a.tokens = m->promptIn;
+            a.seq_len = m->promptIn + r;
+            a.rows = r;
+            a.max_ctx = start + static_cast<uint32_t>(c) + r;
+            a.logits = last ? decode_->logits : nullptr;
+            a.out_token = last ? decode_->out : nullptr;
+            Check(opure_prompt_step(dev_, &a), "opure_prompt_step");
+            c += r;
+            if (last)
+            {
+                int32_t out = 0;
+                Check(opure_buf_download(dev_, &out, decode_->out, 0, 4), "prompt download");
+                return static_cast<uint32_t>(out);
+            }
+        }
+        body = std::max(body, c);
+    }
     if (m->wide)
     {
         // 16 parts of 16 rows a launch, every part at its own offset of the

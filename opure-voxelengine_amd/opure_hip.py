@@ -110,6 +110,11 @@ class VerifyLayerArgs(C.Structure):
                 ("rows", C.c_uint32), ("seq_len", C.c_void_p), ("max_ctx", C.c_uint32), ("x", C.c_void_p)]
 
 
+class PromptArgs(C.Structure):
+    _fields_ = [("model", C.POINTER(Model)), ("kv", C.POINTER(KV)), ("tokens", C.c_void_p), ("seq_len", C.c_void_p),
+                ("rows", C.c_uint32), ("max_ctx", C.c_uint32), ("logits", C.c_void_p), ("out_token", C.c_void_p)]
+
+
 _lib = None
 
 
@@ -153,6 +158,8 @@ def _declare(L):
         "opure_verify_reserve": ([vp, C.POINTER(Model), u32, u32, u32], i),
         "opure_verify_step": ([vp, C.POINTER(VerifyArgs)], i),
         "opure_verify_layer": ([vp, C.POINTER(VerifyLayerArgs)], i),
+        "opure_prompt_reserve": ([vp, C.POINTER(Model), u32, u32], i),
+        "opure_prompt_step": ([vp, C.POINTER(PromptArgs)], i),
         "opure_debug_workspace": ([vp, C.POINTER(vp), C.POINTER(u64)], i),
         "opure_debug_set_wait_limit": ([vp, u32], i),
         "opure_debug_set_gemv_engine": ([vp, u32], i),

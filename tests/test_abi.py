@@ -58,6 +58,7 @@ STRUCTS = {
     "opure_kv": H.KV, "opure_gemv_args": H.GemvArgs, "opure_attn_args": H.AttnArgs,
     "opure_accept_args": H.AcceptArgs, "opure_sample_args": H.SampleArgs,
     "opure_rollback_args": H.RollbackArgs, "opure_verify_args": H.VerifyArgs,
+    "opure_prompt_args": H.PromptArgs,
     "opure_verify_layer_args": H.VerifyLayerArgs,
 }
 

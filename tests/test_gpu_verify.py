@@ -68,6 +68,69 @@ def random_cache(m, B, ctx_max, n_pages, seed):
     return kv
 
 
+@pytest.mark.parametrize("rows,start", [(17, 0), (33, 100), (130, 37), (300, 37), (777, 0)])
+@pytest.mark.parametrize("wfmt,afmt,hd", [(O.W_I8PC, O.A_F16, 64), (O.W_I4G128, O.A_F16, 128), (O.W_I4G128, O.A_BF16, 64)],
+                         ids=["i8-f16-hd64", "i4-f16-hd128", "i4-bf16-hd64"])
+def test_prompt_step_matches_oracle(dev, wfmt, afmt, hd, rows, start):
+    """A prompt of one sequence behind `start` cached positions (a page's
+    middle), up to a batch's rows and past them, with and without K splits:
+    the appended K/V of both layers, the last row's logits and their argmax
+    against the oracle's row by row, within the bars above (bf16: one storage
+    ulp more on K/V, whose values reach past 4); without logits the same K/V."""
+    say("prompt step", wfmt, afmt, hd, rows, start)
+    import npref
+    m = small_model(wfmt, afmt, hd=hd, ffn=2048, attn_scale=hd ** -0.5, tied=wfmt != O.W_I4G128)
+    cap = (start + rows + 16) // 16 * 16
+    kv = random_cache(m, 1, cap, cap // 16 + 3, seed=rows)
+    tokens = np.random.default_rng(rows).integers(0, m.cfg["vocab"], (1, rows)).astype(np.int32)
+    dm = device_model(dev, m)
+    kv_o = O.HostKV(m, n_pages=kv.n_pages, batch=1, max_pages_per_seq=kv.max_pages)
+    kv_o.pool[...], kv_o.page_table[...] = kv.pool, kv.page_table
+    O.set_threads(16)
+    try:
+        want = O.verify_forward(m, kv_o, tokens, np.array([start], np.int32))[0, -1]
+    finally:
+        O.set_threads(1)
+    io = dev.upload(np.concatenate([tokens[0], np.array([start], np.int32)]))
+    lb, ob = dev.alloc(m.cfg["vocab"] * 4), dev.alloc(4)
+    pools = []
+    for logits in (True, False):
+        dkv = device_kv(dev, m, kv)
+        a = H.PromptArgs(C.pointer(dm.desc), C.pointer(dkv.desc), int(io), int(io) + 4 * rows, rows, start + rows,
+                         int(lb) if logits else None, int(ob) if logits else None)
+        H.check(H.lib().opure_prompt_step(dev.h, C.byref(a)))
+        dev.sync()
+        pools.append(dkv.get_pool())
+    got = dev.download(lb, np.float32, (m.cfg["vocab"],))
+    say("max_abs logits", np.abs(got - want).max())
+    assert np.abs(got - want).max() <= 2e-2
+    assert dev.download(ob, np.int32, (1,))[0] == np.argmax(got)
+    g, w = npref.act_to_f32(pools[0], afmt), npref.act_to_f32(kv_o.pool, afmt)
+    assert (np.abs(g - w) <= 2e-2 + (2.0 ** -7 * np.abs(w) if afmt == O.A_BF16 else 0.0)).all()
+    assert np.array_equal(pools[0], pools[1])
+
+
+def test_prompt_step_refuses(dev):
+    """Rows a verify step takes or too many, fp32, another head size, an
+    argmax without logits."""
+    m = small_model(O.W_I8PC, O.A_F16)
+    kv = random_cache(m, 1, 4096, 257, seed=1)
+    for mod, code in (({}, H.OK), ({"rows": 16}, H.E_CAPACITY), ({"rows": 2049}, H.E_CAPACITY), ({"logits": None}, H.E_INVALID),
+                      ({"max_ctx": 31}, H.E_CAPACITY)):
+        dm, dkv = device_model(dev, m), device_kv(dev, m, kv)
+        io, lb = dev.upload(np.zeros(2050, np.int32)), dev.alloc(m.cfg["vocab"] * 4 + 4)
+        v = {"rows": 32, "max_ctx": max(64, mod.get("rows", 0)), "logits": int(lb), **mod}
+        a = H.PromptArgs(C.pointer(dm.desc), C.pointer(dkv.desc), int(io), int(io) + 4 * 2049, v["rows"], v["max_ctx"], v["logits"],
+                         int(lb) + m.cfg["vocab"] * 4)
+        assert H.lib().opure_prompt_step(dev.h, C.byref(a)) == code, mod
+        dev.sync()
+    for m in (small_model(O.W_F32, O.A_F32), small_model(O.W_I8PC, O.A_F16, hd=96)):
+        kv = random_cache(m, 1, 64, 8, seed=1)
+        dm, dkv = device_model(dev, m), device_kv(dev, m, kv)
+        a = H.PromptArgs(C.pointer(dm.desc), C.pointer(dkv.desc), int(io), int(io) + 4 * 2049, 32, 64, None, None)
+        assert H.lib().opure_prompt_step(dev.h, C.byref(a)) == H.E_UNSUPPORTED
+
+
 @pytest.mark.parametrize("fmt", FMTS, ids=FMT_IDS)
 def test_verify_step_matches_oracle(dev, fmt):
     wfmt, afmt, tol = fmt
