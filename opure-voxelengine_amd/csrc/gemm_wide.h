@@ -60,12 +60,19 @@ template <uint32_t TA_, uint32_t TB_, uint32_t WC_, uint32_t KH_> struct WideSha
     static constexpr uint32_t TA = TA_, TB = TB_, WC = WC_, KH = KH_, RT = (4u / WC_) * TA_, CT = WC_ * TB_, NTH = 256u * KH_;
 };
 
-// register slots of the software pipeline: DW weight blocks and DX X blocks
-// in flight; the K loop is unrolled by U = lcm(DW, DX), an even number, so
-// slots and LDS stages are compile-time.
+// The software pipeline goes SB blocks a step (one barrier and one LDS stage a
+// step), DW steps of weights and DX of X in flight in registers; the K loop is
+// unrolled by U steps so slots and stages are compile-time.  At one weight
+// tile a wave a block is 8 or 16 MFMAs behind a barrier, an LDS round trip and
+// the X staging, so two blocks share those; X two steps ahead because loads
+// return in order and a wait for X waits for the weights issued before it (8B layer, 24
+// rows: 131.3 -> 128.5 us).  Eight blocks of weights and four of X in flight
+// were slower (139 us, the loop unrolled eight times), two weight tiles a wave
+// too (1B gate/up at 24 rows 8.8 -> 10.2 us).
 template <int WF, class SH> struct WideDepth {
-    static constexpr bool FEW = SH::CT < 8u, I8 = WF == OPURE_W_I8PC;
-    static constexpr uint32_t DW = I8 ? (SH::KH == 2u ? 4 : 2) : (FEW && SH::TA == 1u ? 4 : 2), DX = I8 ? 2 : (FEW ? 2 : 1), U = DW > DX ? DW : DX;
+    static constexpr bool FEW = SH::TA == 1u, I8 = WF == OPURE_W_I8PC;
+    static constexpr uint32_t SB = FEW ? 2 : 1, DW = !FEW && I8 && SH::KH == 2u ? 4 : 2,
+                              DX = I8 || SH::CT < 8u ? 2 : 1, U = DW > DX ? DW : DX;
 };
 // the plan's splits are multiples of this many blocks
 constexpr uint32_t wide_split_unit(uint32_t wf) { return wf == OPURE_W_I8PC ? 4u : 2u; }
@@ -109,14 +116,14 @@ __global__ __launch_bounds__(SH::NTH) __attribute__((amdgpu_waves_per_eu(2))) vo
     constexpr uint32_t XR = CT * 16u * CH / 256u;  // X chunks a thread stages per block
     constexpr uint32_t STAGE = CT * NMF * 64u;     // u4_t per LDS stage
     using WD = WideDepth<WF, SH>;
-    constexpr uint32_t DW = WD::DW, DX = WD::DX, U = WD::U, KH = SH::KH;
+    constexpr uint32_t SB = WD::SB, DW = WD::DW, DX = WD::DX, U = WD::U, KH = SH::KH;
     static_assert(U % 2 == 0 && U % DX == 0 && U % DW == 0, "static slots and stages");
     constexpr bool GS = WF == OPURE_W_I4G128;      // group sums of X
     static_assert(XR >= 1 && TB % 2 == 0, "whole chunks a thread; the halves exchange half of the column tiles");
     static_assert(KH == 1 || 4u * TA * TB * 64u <= KH * 2u * STAGE, "the halves' exchange reuses the X stages");
     static_assert(!GS || CH == 16u, "a DPP row of lanes stages one X row's group");
-    __shared__ u4_t xl[KH * 2 * STAGE];
-    __shared__ float xsl[GS ? 2 : 1][GS ? CT * 16u : 1u];   // uint4: each stage's group sums of X
+    __shared__ u4_t xl[KH * 2 * SB * STAGE];
+    __shared__ float xsl[GS ? 2 * SB : 1][GS ? CT * 16u : 1u];   // uint4: each block's group sums of X
     const KParams& p = wp.p;
     const uint32_t tid = threadIdx.x & 255u, lane = tid & 63u, g4 = lane >> 4, r16 = lane & 15u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -129,7 +136,7 @@ __global__ __launch_bounds__(SH::NTH) __attribute__((amdgpu_waves_per_eu(2))) vo
     const uint32_t cn = min(wp.cgs, wp.mt - ct0);            // column tiles of this group; of this wave: TB wc + j
     const uint32_t tile0 = rg * RT + wr * TA;
     const uint32_t b_begin = split * wp.bps, b_end = min(nblk, b_begin + wp.bps);
-    u4_t* xh = xl + kh * 2u * STAGE;                          // this half's two stages
+    u4_t* xh = xl + kh * 2u * SB * STAGE;                     // this half's two stages of SB blocks
 
     // X chunk u of this thread: row rr of local column tile ctl, 16-byte chunk c of the block (a
     // wave's load covers 8 rows x 128 contiguous bytes).  In LDS, chunk c of row rr sits at row
@@ -308,26 +315,36 @@ __global__ __launch_bounds__(SH::NTH) __attribute__((amdgpu_waves_per_eu(2))) vo
     }
 
     // Half kh takes blocks b_begin + kh, + kh + KH, ...; a step moves both
-    // halves one block on, with one barrier for the whole workgroup.
-    const uint32_t steps = (b_end - b_begin + KH - 1u) / KH;
+    // halves SB blocks on, with one barrier for the whole workgroup.
+    const uint32_t steps = (b_end - b_begin + KH * SB - 1u) / (KH * SB);
     const uint32_t bh = b_begin + kh;
-    u4_t xr[DX][XR];
-    u4_t wv[DW][TA], sv[DW][TA];
+    u4_t xr[DX][SB][XR];
+    u4_t wv[DW][SB][TA], sv[DW][SB][TA];
+    auto block = [&](uint32_t step, uint32_t k) { return bh + KH * (SB * step + k); };
 #pragma unroll
-    for (uint32_t d = 0; d < DX; ++d) xload(xr[d], bh + KH * d);
+    for (uint32_t d = 0; d < DX; ++d)
 #pragma unroll
-    for (uint32_t d = 0; d < DW; ++d) wload(wv[d], sv[d], bh + KH * d);
+        for (uint32_t k = 0; k < SB; ++k) xload(xr[d][k], block(d, k));
+#pragma unroll
+    for (uint32_t d = 0; d < DW; ++d)
+#pragma unroll
+        for (uint32_t k = 0; k < SB; ++k) wload(wv[d][k], sv[d][k], block(d, k));
     for (uint32_t i0 = 0; i0 < steps; i0 += U)
     {
 #pragma unroll
         for (uint32_t s = 0; s < U; ++s)
         {
-            const uint32_t b = bh + KH * (i0 + s);
-            xstore(xr[s % DX], s & 1u);
-            xload(xr[s % DX], b + KH * DX);
+            const uint32_t st = (s & 1u) * SB;
+#pragma unroll
+            for (uint32_t k = 0; k < SB; ++k) xstore(xr[s % DX][k], st + k);
+#pragma unroll
+            for (uint32_t k = 0; k < SB; ++k) xload(xr[s % DX][k], block(i0 + s + DX, k));
             __syncthreads();
-            if (b < b_end) compute(wv[s % DW], sv[s % DW], s & 1u);
-            wload(wv[s % DW], sv[s % DW], b + KH * DW);
+#pragma unroll
+            for (uint32_t k = 0; k < SB; ++k)
+                if (block(i0 + s, k) < b_end) compute(wv[s % DW][k], sv[s % DW][k], st + k);
+#pragma unroll
+            for (uint32_t k = 0; k < SB; ++k) wload(wv[s % DW][k], sv[s % DW][k], block(i0 + s + DW, k));
         }
     }
 
