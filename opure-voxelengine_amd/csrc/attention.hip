@@ -702,8 +702,13 @@ __device__ __forceinline__ float unpack_hi(uint32_t v)
 template <int AF>
 __device__ __forceinline__ uint32_t pack_pair(float a, float b)
 {
-    if constexpr (AF == OPURE_A_F16) return f32_to_f16(a) | (static_cast<uint32_t>(f32_to_f16(b)) << 16);
-    else return f32_to_bf16(a) | (static_cast<uint32_t>(f32_to_bf16(b)) << 16);
+    // one v_cvt_pk_f16_f32 / v_cvt_pk_bf16_f32, round to nearest even
+    typedef float f2v __attribute__((ext_vector_type(2)));
+    typedef _Float16 h2v __attribute__((ext_vector_type(2)));
+    typedef __bf16 b2v __attribute__((ext_vector_type(2)));
+    const f2v v = {a, b};
+    if constexpr (AF == OPURE_A_F16) return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, h2v));
+    else return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, b2v));
 }
 
 // Matrix-core flash-decoding for fp16/bf16 caches, head_dim HD in {64, 128}.
@@ -934,10 +939,20 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(CL ? 4
                 }
             }
         }
+        // a wave whose tokens every row sees, all on pages that are there, skips
+        // the fills and the masks (most waves of a long context)
+        bool full = tw + TPW <= ctx + 1u;
+        if constexpr (CL)
+        {
+            bool ok = true;
+#pragma unroll
+            for (uint32_t kk = 0; kk < KK; ++kk) ok = ok && kok[kk][0] && kok[kk][1] && vok[kk];
+            full = full && __all(ok);
+        }
         // the folded kernel's operands as used: the fill where the page is
         // missing, and V's slots past the cache read 0
         auto fix_k = [&](uint32_t kk) {
-            if constexpr (CL)
+            if (CL && !full)
 #pragma unroll
                 for (uint32_t T = 0; T < 2; ++T)
 #pragma unroll
@@ -948,7 +963,7 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(CL ? 4
                     }
         };
         auto fix_v = [&](uint32_t kk) {
-            if constexpr (CL)
+            if (CL && !full)
             {
                 const uint32_t f = vfill[kk];
 #pragma unroll
@@ -970,7 +985,6 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(CL ? 4
 #pragma unroll
         for (uint32_t kk = 0; kk < KK; ++kk)
         {
-            const uint32_t tb = tw + 32u * kk;
             fix_k(kk);
 #pragma unroll
             for (uint32_t T = 0; T < 2; ++T)
@@ -981,13 +995,19 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(CL ? 4
 #pragma unroll
                     for (uint32_t s = 0; s < KS; ++s) acc = mfma32<AF>(kop[kk][T][s], qop[n][s], acc);
 #pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                    {
-                        const uint32_t tok = tb + 8u * g + 4u * T + i;
-                        sc[kk][T][n][i] = active && tok <= lim[n] ? __fmul_rn(acc[i], p.scale) : -__builtin_huge_valf();
-                    }
+                    for (int i = 0; i < 4; ++i) sc[kk][T][n][i] = __fmul_rn(acc[i], p.scale);
                 }
         }
+        if (!full)
+#pragma unroll
+            for (uint32_t kk = 0; kk < KK; ++kk)
+#pragma unroll
+                for (uint32_t T = 0; T < 2; ++T)
+#pragma unroll
+                    for (int n = 0; n < NT; ++n)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            if (!active || tw + 32u * kk + 8u * g + 4u * T + i > lim[n]) sc[kk][T][n][i] = -__builtin_huge_valf();
 
         // ---- softmax statistics of each query row over this wave's tokens -----
         // P^T = hi + lo (fp16) or hi + mid + lo (bf16), every part in the 16-bit format
@@ -1100,7 +1120,7 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(CL ? 4
         float ew[NWV];
 #pragma unroll
         for (int w = 0; w < NWV; ++w)
-            ew[w] = mw[w] == -__builtin_huge_valf() ? 0.0f : expf_ref_nonpos(__fsub_rn(mw[w], M));
+            ew[w] = mw[w] == -__builtin_huge_valf() ? 0.0f : exp_hw(__fsub_rn(mw[w], M));
         float L = __fmul_rn(ew[0], lw[0]);
 #pragma unroll
         for (int w = 1; w < NWV; ++w) L = __fmaf_rn(ew[w], lw[w], L);
