@@ -431,8 +431,10 @@ __global__ __launch_bounds__(256) void k_wide_reduce(WParams wp)
 // (g0 + g1) + (g2 + g3) -- then inv_rms from the tile sums in inv_rms_wave's
 // order and round(y * inv * gain) as k_rmsnorm_rows, so y, ss_out and the
 // normalised rows equal the separate passes' bit for bit.
-constexpr uint32_t RN_THREADS = 256, RN_SPLITS = 8;   // the plan splits K at most 8 ways
-template <int WF, int AF, int UNITS>
+// RN_THREADS 1024 for batches of fewer rows than CUs, 256 past that: a few rows
+// are one round trip of each thread's loads, so fewer a thread.
+constexpr uint32_t RN_SPLITS = 8;   // the plan splits K at most 8 ways
+template <int WF, int AF, int UNITS, uint32_t RN_THREADS>
 __global__ __launch_bounds__(RN_THREADS) void k_wide_reduce_norm(WParams wp, const float* gain, void* xn)
 {
     const KParams& p = wp.p;
@@ -510,14 +512,16 @@ __global__ __launch_bounds__(RN_THREADS) void k_wide_reduce_norm(WParams wp, con
     }
 }
 
-// outputs up to 2048 (2 units of 4 a thread) or 4096 (4)
+// outputs up to 2048 (2 units of 4 a thread of 256) or 4096 (4, or 1 of 1024)
 template <int WF, int AF>
 int launch_wide_reduce_norm(opure_dev* dev, const WParams& wp, const float* gain, void* xn)
 {
-    if (wp.p.out <= 8u * RN_THREADS)
-        OPURE_LAUNCH(dev, (k_wide_reduce_norm<WF, AF, 2>), dim3(wp.p.M), dim3(RN_THREADS), 0, wp, gain, xn);
+    if (wp.p.M <= 128u)
+        OPURE_LAUNCH(dev, (k_wide_reduce_norm<WF, AF, 1, 1024u>), dim3(wp.p.M), dim3(1024), 0, wp, gain, xn);
+    else if (wp.p.out <= 2048u)
+        OPURE_LAUNCH(dev, (k_wide_reduce_norm<WF, AF, 2, 256u>), dim3(wp.p.M), dim3(256), 0, wp, gain, xn);
     else
-        OPURE_LAUNCH(dev, (k_wide_reduce_norm<WF, AF, 4>), dim3(wp.p.M), dim3(RN_THREADS), 0, wp, gain, xn);
+        OPURE_LAUNCH(dev, (k_wide_reduce_norm<WF, AF, 4, 256u>), dim3(wp.p.M), dim3(256), 0, wp, gain, xn);
     OPURE_LAUNCH_CHECK("k_wide_reduce_norm");
     return OPURE_OK;
 }

@@ -122,6 +122,60 @@ __global__ __launch_bounds__(256) void k_tile_sumsq(const float* x, uint32_t M, 
     ss[static_cast<uint64_t>(c16) * M + r] = sq;
 }
 
+// k_tile_sumsq and the rmsnorm rows pass (gemv.hip) in one: a workgroup a row,
+// a thread a 16-column tile (h <= 4096), the tile sums in inv_rms_wave's order,
+// round(x * inv * gain) -- the bits of the two launches.  For the layer that
+// starts from a caller's residual over more than OPURE_MAX_ROWS rows.
+template <int AF>
+__global__ __launch_bounds__(256) void k_norm_rows(const float* x, const float* gain, uint32_t h, float eps, void* xn)
+{
+    typedef float f4v __attribute__((ext_vector_type(4)));
+    typedef uint32_t u4v __attribute__((ext_vector_type(4)));
+    __shared__ float ss[256];
+    const uint32_t tiles = h / 16u, t = threadIdx.x, lane = t & 63u;
+    const bool live = t < tiles;
+    const uint32_t c = 16u * min(t, tiles - 1u);
+    const float* xr = x + static_cast<uint64_t>(blockIdx.x) * h + c;
+    float v[16], g[16];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+    {
+        const f4v a = reinterpret_cast<const f4v*>(xr)[q], b = reinterpret_cast<const f4v*>(gain + c)[q];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+        {
+            v[4 * q + e] = a[e];
+            g[4 * q + e] = b[e];
+        }
+    }
+    float sq = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) sq = __fmaf_rn(v[e], v[e], sq);
+    ss[t] = sq;
+    __syncthreads();
+    float sum = 0.0f;
+    for (uint32_t i = lane; i < tiles; i += 64u) sum += ss[i];
+    sum = row16_sum(sum);
+    sum = add_xor32(add_xor16(sum));
+    const float inv = __fdiv_rn(1.0f, __fsqrt_rn(__fadd_rn(__fdiv_rn(sum, static_cast<float>(h)), eps)));
+    if (!live) return;
+    typedef float f2v __attribute__((ext_vector_type(2)));
+    typedef _Float16 h2v __attribute__((ext_vector_type(2)));
+    typedef __bf16 b2v __attribute__((ext_vector_type(2)));
+    uint32_t o[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+    {
+        // narrowed as pairs: a product narrowed alone may round once instead of twice
+        const f2v y = {__fmul_rn(__fmul_rn(v[2 * i], inv), g[2 * i]), __fmul_rn(__fmul_rn(v[2 * i + 1], inv), g[2 * i + 1])};
+        o[i] = AF == OPURE_A_F16 ? __builtin_bit_cast(uint32_t, __builtin_convertvector(y, h2v))
+                                 : __builtin_bit_cast(uint32_t, __builtin_convertvector(y, b2v));
+    }
+    u4v* dst = reinterpret_cast<u4v*>(static_cast<uint16_t*>(xn) + static_cast<uint64_t>(blockIdx.x) * h + c);
+    dst[0] = u4v{o[0], o[1], o[2], o[3]};
+    dst[1] = u4v{o[4], o[5], o[6], o[7]};
+}
+
 // the position of a prompt's last row
 __global__ void k_last_position(const int32_t* seq_len, uint32_t rows, int32_t* out)
 {
@@ -474,11 +528,21 @@ int opure_verify_layer(opure_dev* dev, const opure_verify_layer_args* a)
     if ((rc = ensure_workspace(dev, P.total))) return rc;
     char* ws = static_cast<char*>(dev->ws);
     float* ss = reinterpret_cast<float*>(ws + P.ss);
+    GemvCall c = step_gemv(m, MR, P, ws, ss);
+    // 16-bit rows of more than a GEMV's: the normalised rows at once
+    if (MR > OPURE_MAX_ROWS && m->hidden <= 4096u && m->afmt != OPURE_A_F32 && (reinterpret_cast<uintptr_t>(a->x) & 15u) == 0u &&
+        (reinterpret_cast<uintptr_t>(m->layers[a->layer].attn_norm) & 15u) == 0u)
+    {
+        const float* gain = m->layers[a->layer].attn_norm;
+        if (m->afmt == OPURE_A_F16) OPURE_LAUNCH(dev, k_norm_rows<OPURE_A_F16>, dim3(MR), dim3(256), 0, a->x, gain, m->hidden, m->rms_eps, ws + P.xn);
+        else OPURE_LAUNCH(dev, k_norm_rows<OPURE_A_BF16>, dim3(MR), dim3(256), 0, a->x, gain, m->hidden, m->rms_eps, ws + P.xn);
+        OPURE_LAUNCH_CHECK("k_norm_rows");
+        return layer_launch(dev, m, a->kv, a->layer, B, R, a->seq_len, a->max_ctx, P, a->x, ss, c, true);
+    }
     const uint64_t n = static_cast<uint64_t>(MR) * (m->hidden / 16u);
     OPURE_LAUNCH(dev, k_tile_sumsq, dim3(static_cast<uint32_t>((n + 255u) / 256u)), dim3(256), 0, a->x, MR,
                        m->hidden, ss);
     OPURE_LAUNCH_CHECK("k_tile_sumsq");
-    GemvCall c = step_gemv(m, MR, P, ws, ss);
     return layer_launch(dev, m, a->kv, a->layer, B, R, a->seq_len, a->max_ctx, P, a->x, ss, c);
 }
 

@@ -68,6 +68,37 @@ def random_cache(m, B, ctx_max, n_pages, seed):
     return kv
 
 
+@pytest.mark.parametrize("hidden", [192, 1088, 4096, 4160])
+@pytest.mark.parametrize("afmt", [O.A_F16, O.A_BF16], ids=["f16", "bf16"])
+def test_layer_norm_rows_same_bits(dev, hidden, afmt):
+    """opure_verify_layer over more than 16 rows normalises its residual in one
+    launch (hidden up to 4096, past that in two): from the embedding rows its
+    first layer appends the K/V that the whole step (whose embedding leaves the
+    tile sums) appends, bit for bit."""
+    if afmt == O.A_BF16:
+        hidden = (hidden + 127) // 128 * 128
+    say("layer norm rows", hidden, afmt)
+    wfmt = O.W_I8PC if afmt == O.A_F16 else O.W_I4G128
+    m = small_model(wfmt, afmt, n_layers=1, hidden=hidden, ffn=256, vocab=64, tied=wfmt != O.W_I4G128)
+    B, R = 7, 3
+    kv = random_cache(m, B, 48, B * 3 + 2, seed=hidden)
+    tokens = np.random.default_rng(hidden).integers(0, 64, (B, R)).astype(np.int32)
+    ctx = np.array([0, 5, 13, 14, 15, 30, 40], np.int32)
+    dm = device_model(dev, m)
+    pools = []
+    dkv = device_kv(dev, m, kv)
+    run = VerifyRunner(dev, dm, dkv, B, R, max_ctx=48)
+    run.step(tokens, ctx)
+    pools.append(dkv.get_pool())
+    dkv = device_kv(dev, m, kv)
+    x, sl = dev.upload(O.verify_embed(m, tokens)), dev.upload(ctx)
+    a = H.VerifyLayerArgs(C.pointer(dm.desc), C.pointer(dkv.desc), 0, B, R, int(sl), 48, int(x))
+    H.check(H.lib().opure_verify_layer(dev.h, C.byref(a)))
+    dev.sync()
+    pools.append(dkv.get_pool())
+    assert np.array_equal(pools[0], pools[1]) and not np.array_equal(pools[0], kv.pool)
+
+
 @pytest.mark.parametrize("rows,start", [(17, 0), (33, 100), (130, 37), (300, 37), (777, 0)])
 @pytest.mark.parametrize("wfmt,afmt,hd", [(O.W_I8PC, O.A_F16, 64), (O.W_I4G128, O.A_F16, 128), (O.W_I4G128, O.A_BF16, 64)],
                          ids=["i8-f16-hd64", "i4-f16-hd128", "i4-bf16-hd64"])
