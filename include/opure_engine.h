@@ -17,8 +17,8 @@
  *  array of layer descriptors must outlive it) and owns its KV pools, page
  *  tables, step buffers and captured graphs.  Each model's KV pool is a set of
  *  16-token pages handed out by a free list as the sequence grows and given
- *  back by the rollback; prompts of quantised models are prefilled 256 rows a
- *  launch.
+ *  back by the rollback; prompts of quantised models are prefilled up to
+ *  2,048 tokens a step (256 at head sizes other than 64 and 128).
  * ========================================================================== */
 #ifndef OPURE_ENGINE_H
 #define OPURE_ENGINE_H

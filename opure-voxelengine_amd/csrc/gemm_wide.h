@@ -1,6 +1,7 @@
 // ============================================================================
 //  gemm_wide.h -- the GEMV for more than 16 activation rows (a batch of
-//  sequences times K+1 rows, up to 256): a thin GEMM on the matrix cores.
+//  sequences times K+1 rows, up to 256, or a prompt's, up to 2,048): a thin
+//  GEMM on the matrix cores.
 //
 //  The same tiled weights and the same MFMA operand mapping as the K+1-row
 //  kernel (gemv_kernel.h): y^T = W X^T in 16 x 16 tiles, A = 16 weight rows
@@ -12,8 +13,9 @@
 //  set of 4 waves covers the row group (more than 64 rows of X): wave w multiplies
 //  tiles 2w, 2w + 1 by all of the group's column tiles, so it keeps 16 accumulator
 //  tiles, loads each weight byte once and reads each B fragment once per block for
-//  two MFMAs.  Fewer rows take one weight tile a wave (WideShape).  Weights go straight from HBM into registers: every wave loads its
-//  own two tiles' 16 bytes a lane per block, in static register slots DW
+//  two MFMAs.  Fewer rows take one weight tile a wave, a prompt's
+//  rows four on a 2 x 2 wave grid (WideShape).  Weights go straight from HBM into
+//  registers: every wave loads its own tiles' 16 bytes a lane per block, in static register slots DW
 //  blocks ahead.  X goes through LDS: per block the set loads its column
 //  group's fragments into registers DX blocks ahead and writes them into a
 //  two-stage ring laid out fragment by fragment, 16 bytes a lane.  One barrier
@@ -43,7 +45,6 @@ namespace opure_gemv {
 
 constexpr uint32_t WIDE_RT = 8;       // weight tiles of the plan's row groups (the K splits follow from these)
 constexpr uint32_t WIDE_CG = 8;       // column tiles per workgroup at most
-constexpr uint32_t WIDE_MAX_M = 256;  // rows of X
 
 // The wave grid: a set of 4 waves is 4 / WC wave rows x WC wave columns, each
 // wave TA weight tiles x TB column tiles.  CT = WC * TB column tiles a
@@ -65,8 +66,8 @@ template <uint32_t TA_, uint32_t TB_, uint32_t WC_, uint32_t KH_> struct WideSha
 // unrolled by U steps so slots and stages are compile-time.  At one weight
 // tile a wave a block is 8 or 16 MFMAs behind a barrier, an LDS round trip and
 // the X staging, so two blocks share those; X two steps ahead because loads
-// return in order and a wait for X waits for the weights issued before it (8B layer, 24
-// rows: 131.3 -> 128.5 us).  Eight blocks of weights and four of X in flight
+// return in order and a wait for X waits for the weights issued before it (8B layer,
+// 24 rows: 131.3 -> 128.5 us).  Eight blocks of weights and four of X in flight
 // were slower (139 us, the loop unrolled eight times), two weight tiles a wave
 // too (1B gate/up at 24 rows 8.8 -> 10.2 us).
 template <int WF, class SH> struct WideDepth {

@@ -19,11 +19,12 @@
 //
 //  Each model's KV cache is a pool of 16-token pages handed out by a PagePool:
 //  a sequence's page-table row takes pages as it grows (before a step writes
-//  there) and the rollback's freed pages go back to the pool.  Prompts are
-//  prefilled 256 rows a launch where the weights are quantised and the
-//  activations 16-bit: one verify step over 16 "sequences" of 16 rows that
-//  share the prompt's page-table row (row j of part b sits at start + 16 b + j
-//  and sees every position before it), so every GEMV runs as a thin GEMM.
+//  there) and the rollback's freed pages go back to the pool.  Prompts of
+//  quantised weights and 16-bit activations go through opure_prompt_step, up to
+//  2,048 tokens a step, the last of which leaves the next token and its logits;
+//  at head sizes that step is not built for, 256 rows a launch: one verify step
+//  over 16 "sequences" of 16 rows that share the prompt's page-table row (row j
+//  of part b sits at start + 16 b + j and sees every position before it).
 // ============================================================================
 #pragma once
 
