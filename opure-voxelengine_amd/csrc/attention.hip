@@ -481,14 +481,15 @@ __global__ __launch_bounds__(attn_fast_threads<HD>()) void k_attn_chunk(AttnPara
 // context): a workgroup per (KV head, pair of query rows, sequence) with a
 // wave per chunk, so a batch of one sequence still spreads over many CUs.  A
 // wave loads its chunk's K rows (lane = token) and V columns (lane = channel)
-// straight into registers, all at once (a missing page's lanes read page 0
+// into registers, all at once (a missing page's lanes read page 0
 // and are replaced when used), scores the pair of rows with the chunk
 // kernel's per-row operations and leaves the chunk's (max, sum, output) in
 // LDS; the waves then merge each row's chunks with k_attn_combine's
 // operations in its order.  A row has the bits of k_attn_chunk + combine.
 constexpr uint32_t ATTN_SPLIT_CHUNKS = 8;
+constexpr uint32_t attn_split_lds(uint32_t chunks) { return chunks * 64u * (64u * 4u + 16u); }
 
-template <int AF>
+template <int AF, bool TURN>
 __global__ __launch_bounds__(64 * ATTN_SPLIT_CHUNKS) void k_attn_split(AttnParams p)
 {
     constexpr uint32_t HD = 64, CH = 64, RB = 2, NW = ATTN_SPLIT_CHUNKS, PPC = CH / OPURE_PAGE_SIZE;
@@ -498,6 +499,7 @@ __global__ __launch_bounds__(64 * ATTN_SPLIT_CHUNKS) void k_attn_split(AttnParam
     __shared__ __align__(16) float pa[NW][RB][HD];        // the chunks' outputs
     __shared__ float pm[NW][RB], pl[NW][RB];               // the chunks' maxima and sums
     __shared__ float wsh[RB][NW];                          // a row's chunk weights
+    extern __shared__ __align__(16) uint8_t tile_lds[];    // a wave's K, then V tile (attn_split_lds)
 
     const uint32_t kh = blockIdx.x, b = blockIdx.z;
     const uint32_t group = p.n_heads / p.n_kv, R = p.rows, Gq = group * R;
@@ -531,25 +533,80 @@ __global__ __launch_bounds__(64 * ATTN_SPLIT_CHUNKS) void k_attn_split(AttnParam
 
     if (t0 < total)   // wave-uniform: the chunk holds positions of the sequence
     {
-        // round trip 2: K row of token t0 + lane, V column of channel `lane`
+        // round trip 2: K row of token t0 + lane, V column of channel `lane`,
+        // each lane its own, or (TURN) the chunk's pages in memory order, a wave
+        // instruction 1 KB of a plane, then the same through the wave's LDS in
+        // rows padded by a piece
         auto ok = [&](int32_t pg_) { return pg_ >= 0 && static_cast<uint32_t>(pg_) < p.n_pages; };
         auto safe = [&](int32_t pg_) { return ok(pg_) ? static_cast<uint32_t>(pg_) : 0u; };
         const uint32_t pos = t0 + lane, sl = lane / OPURE_PAGE_SIZE;
         const int32_t kpg = sl == 0u ? pg[0] : sl == 1u ? pg[1] : sl == 2u ? pg[2] : pg[3];
-        const u4v* kp = reinterpret_cast<const u4v*>(static_cast<const uint8_t*>(p.pool) +
-                                                     kv_elem(p.layer, p.n_pages, safe(kpg), 0u, p.n_kv, kh, HD,
-                                                             pos % OPURE_PAGE_SIZE, 0u) * EB);
+        static_assert(AF == OPURE_A_F32, "pieces of four values");
         u4v kw[HD / EPP], vw[PPC][OPURE_PAGE_SIZE / EPP];
+        if constexpr (!TURN)
+        {
+            const u4v* kp = reinterpret_cast<const u4v*>(static_cast<const uint8_t*>(p.pool) +
+                                                         kv_elem(p.layer, p.n_pages, safe(kpg), 0u, p.n_kv, kh, HD,
+                                                                 pos % OPURE_PAGE_SIZE, 0u) * EB);
 #pragma unroll
-        for (uint32_t k = 0; k < HD / EPP; ++k) kw[k] = kp[k];
+            for (uint32_t k = 0; k < HD / EPP; ++k) kw[k] = kp[k];
+#pragma unroll
+            for (uint32_t i = 0; i < PPC; ++i)
+            {
+                const u4v* vp = reinterpret_cast<const u4v*>(static_cast<const uint8_t*>(p.pool) +
+                                                             kv_elem(p.layer, p.n_pages, safe(pg[i]), 1u, p.n_kv, kh, HD, 0u,
+                                                                     lane) * EB);
+#pragma unroll
+                for (uint32_t k = 0; k < OPURE_PAGE_SIZE / EPP; ++k) vw[i][k] = vp[k];
+            }
+        }
+        else
+        {
+        constexpr uint32_t ROW = HD * EB + 16u, PLN = OPURE_PAGE_SIZE * HD * EB / 1024u;   // LDS row bytes; loads a plane
+        uint8_t* tl = tile_lds + c * CH * ROW;
+        u4v kraw[PPC][PLN], vraw[PPC][PLN];
 #pragma unroll
         for (uint32_t i = 0; i < PPC; ++i)
         {
-            const u4v* vp = reinterpret_cast<const u4v*>(static_cast<const uint8_t*>(p.pool) +
-                                                         kv_elem(p.layer, p.n_pages, safe(pg[i]), 1u, p.n_kv, kh, HD, 0u,
-                                                                 lane) * EB);
+            const uint8_t* kp = static_cast<const uint8_t*>(p.pool) + kv_elem(p.layer, p.n_pages, safe(pg[i]), 0u, p.n_kv, kh, HD, 0u, 0u) * EB;
+            const uint8_t* vp = static_cast<const uint8_t*>(p.pool) + kv_elem(p.layer, p.n_pages, safe(pg[i]), 1u, p.n_kv, kh, HD, 0u, 0u) * EB;
 #pragma unroll
-            for (uint32_t k = 0; k < OPURE_PAGE_SIZE / EPP; ++k) vw[i][k] = vp[k];
+            for (uint32_t k = 0; k < PLN; ++k)
+            {
+                kraw[i][k] = *reinterpret_cast<const u4v*>(kp + (k * 64u + lane) * 16u);
+                vraw[i][k] = *reinterpret_cast<const u4v*>(vp + (k * 64u + lane) * 16u);
+            }
+        }
+        auto wave_sync = [] {
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        };
+#pragma unroll
+        for (uint32_t i = 0; i < PPC; ++i)
+#pragma unroll
+            for (uint32_t k = 0; k < PLN; ++k)
+            {
+                const uint32_t e = k * 64u + lane;                     // piece of the plane: token e / 16
+                *reinterpret_cast<u4v*>(tl + (OPURE_PAGE_SIZE * i + e / (HD / EPP)) * ROW + (e % (HD / EPP)) * 16u) = kraw[i][k];
+            }
+        wave_sync();
+#pragma unroll
+        for (uint32_t k = 0; k < HD / EPP; ++k) kw[k] = *reinterpret_cast<const u4v*>(tl + lane * ROW + k * 16u);
+        wave_sync();
+#pragma unroll
+        for (uint32_t i = 0; i < PPC; ++i)
+#pragma unroll
+            for (uint32_t k = 0; k < PLN; ++k)
+            {
+                const uint32_t e = k * 64u + lane;                     // channel e / 4, four tokens
+                *reinterpret_cast<u4v*>(tl + (e / 4u) * ROW + OPURE_PAGE_SIZE * EB * i + (e % 4u) * 16u) = vraw[i][k];
+            }
+        wave_sync();
+#pragma unroll
+        for (uint32_t i = 0; i < PPC; ++i)
+#pragma unroll
+            for (uint32_t k = 0; k < OPURE_PAGE_SIZE / EPP; ++k)
+                vw[i][k] = *reinterpret_cast<const u4v*>(tl + lane * ROW + OPURE_PAGE_SIZE * EB * i + k * 16u);
         }
         // the fills: a position past the cache reads 0, a missing page (or an
         // entry past the table) NaN, a V piece reaching past the cache keeps
@@ -1937,7 +1994,24 @@ int attn_launch(opure_dev* dev, const opure_model* m, const opure_kv* kv, uint32
         // a short context at head_dim 64: a workgroup a pair of query rows, a
         // wave a chunk, merged in the workgroup (no combine launch)
         const dim3 g(p.n_kv, (Gq + 1u) / 2u, batch), blk(64u * p.nch);
-        OPURE_LAUNCH(dev, k_attn_split<OPURE_A_F32>, g, blk, 0, p);
+        // past 4 chunks (one workgroup a CU by its registers either way) K and V
+        // are loaded in memory order and turned in LDS: a lane's own row is a
+        // 64-byte access a lane, 2,048 clocks a wave (3 KV heads, 5 rows: 300
+        // tokens 8.6 -> 7.8 us, 490 10.3 -> 8.4).  Up to 4 the tiles' LDS would
+        // take a CU's second workgroup (12 sequences of 200 tokens 13.3 -> 18.3).
+        if (p.nch > 4u)
+        {
+            static bool configured = false;
+            if (!configured)
+            {
+                OPURE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_attn_split<OPURE_A_F32, true>),
+                                                  hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                  static_cast<int>(attn_split_lds(ATTN_SPLIT_CHUNKS))));
+                configured = true;
+            }
+            OPURE_LAUNCH(dev, (k_attn_split<OPURE_A_F32, true>), g, blk, attn_split_lds(p.nch), p);
+        }
+        else OPURE_LAUNCH(dev, (k_attn_split<OPURE_A_F32, false>), g, blk, 0, p);
         OPURE_LAUNCH_CHECK("k_attn_split");
         return OPURE_OK;
     }
