@@ -624,6 +624,52 @@ def test_attention_every_head_size(dev, afmt, hd):
         x.free()
 
 
+def split_act(x, afmt, n):
+    """x as n values of the storage format, each the rounding of what the ones
+    before leave."""
+    parts = []
+    for _ in range(n):
+        v = float(to_act(np.float32(x), afmt)[1])
+        parts.append(v)
+        x -= v
+    return parts
+
+
+@pytest.mark.parametrize("hd", [64, 96, 128])
+@pytest.mark.parametrize("afmt", [H.A_F16, H.A_BF16], ids=["f16", "bf16"])
+def test_attention_wave_merge_weights(dev, afmt, hd):
+    """A wave's weight in the merge of a chunk is expf_ref of its maximum less
+    the chunk's, to the bit.  Wave 0's tokens score 0 and wave 1's -x, so every
+    probability is 1 and the output is (S0 + e^-x S1) / (n + n e^-x); S0 cancels
+    e^-x S1 but for its last bits, which is what the stored output then holds."""
+    say("wave merge weights", hd, afmt)
+    n = 64 if hd == 128 else 32                    # tokens a wave
+    xs = [to_act(np.float32(v), afmt)[1].item() for v in np.linspace(0.3, 9.0, 24)]
+    B, pages = len(xs), 2 * n // 16
+    K, V = np.zeros((B, 2 * n, hd), np.float32), np.zeros((B, 2 * n, hd), np.float32)
+    want = np.zeros(B, np.float32)
+    f32 = np.float32
+    for b, x in enumerate(xs):
+        e = f32(O.lib().orc_expf(-x))
+        s1 = 32768.0
+        s0 = [-v for v in split_act(float(e) * s1, afmt, 2 if afmt == H.A_F16 else 3)]
+        K[b, n:, 0] = -x
+        V[b, :len(s0)] = np.array(s0)[:, None]
+        V[b, n:] = s1 / n
+        a = f32(float(e) * s1 + sum(s0))           # one fma: exact, then rounded
+        L = f32(float(e) * n + n)
+        want[b] = f32(a / L)
+    k_bits, v_bits = to_act(K, afmt)[0], to_act(V, afmt)[0]
+    pool = np.zeros((1, B * pages, 2, 1, 16 * hd), np.uint16)
+    pool[0, :, 0, 0] = k_bits.reshape(B * pages, 16 * hd)
+    pool[0, :, 1, 0] = v_bits.reshape(B * pages, 16, hd).transpose(0, 2, 1).reshape(B * pages, 16 * hd)
+    pt = np.arange(B * pages, dtype=np.int32).reshape(B, pages)
+    q = np.zeros((B, hd), np.float32)
+    q[:, 0] = 1.0
+    got = run_attn(dev, attn_model(1, 1, hd, afmt), pool, pt, [2 * n - 1] * B, 1, to_act(q, afmt)[0])
+    assert np.array_equal(got, np.repeat(to_act(want, afmt)[0][:, None], hd, 1))
+
+
 # fp32 launches over few chunks of 64 tokens: head_dim, query heads, KV heads,
 # rows, contexts (rows ending on either side of chunk boundaries)
 FAST_ALL_CASES = [
