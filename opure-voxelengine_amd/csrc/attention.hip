@@ -26,9 +26,9 @@
 //  2^-25 relative, where one bf16 operand would give 8 bits).  A bf16 model
 //  rounds the attention output to 8 bits next, and any difference from the
 //  exactly summed softmax moves some of those roundings.  Other head sizes run
-//  on the same kernel with 128-token chunks (32 heads of 96, 4 sequences of 5
-//  rows up to 1,500 tokens: 43.8 us on the VALU, 7.7 us here).  fp32 caches use
-//  VALU kernels.
+//  on the same kernel with 128-token chunks and probabilities of 24 bits in both
+//  formats (32 heads of 96, 4 sequences of 5 rows up to 1,500 tokens, with the
+//  combine: 53 us on the VALU, 11.9 us here).  fp32 caches use VALU kernels.
 // ============================================================================
 #include "internal.h"
 
@@ -834,7 +834,11 @@ __device__ __forceinline__ float merge_val(float sa, float a, float sb, float c)
 // CL: a workgroup takes the ATTN_GROUP chunks from ATTN_GROUP * blockIdx.y and
 //     writes their merge as partial blockIdx.y
 // RH: the head size is p.hd = HD or HD - 16 (every multiple of 16 that is not 64
-//     or 128): channels past it read 0 in K and Q, their V tile is left out
+//     or 128): channels past it read 0 in K and Q, their V tile is left out.
+//     These head sizes keep what the vector kernel gives them: probabilities of
+//     24 bits from expf_ref.  Three 16-bit parts hold those; fp16's are those of
+//     2^15 P, as those of P would end at 2^-24, a bit short of P itself below
+//     1/2 (2^15 P and 65,504 times it stay far inside fp32).
 template <int HD, int AF, int NT, int KK, int NWV, bool ZS, bool CL = false, bool RH = false>
 __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(CL ? 4 : 1))) void k_attn_mfma(AttnParams p)
 {
@@ -1067,8 +1071,10 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(CL ? 4
                             if (!active || tw + 32u * kk + 8u * g + 4u * T + i > lim[n]) sc[kk][T][n][i] = -__builtin_huge_valf();
 
         // ---- softmax statistics of each query row over this wave's tokens -----
-        // P^T = hi + lo (fp16) or hi + mid + lo (bf16), every part in the 16-bit format
-        constexpr bool P3 = AF == OPURE_A_BF16;
+        // P^T = hi + lo (fp16) or hi + mid + lo (bf16), every part in the 16-bit
+        // format; RH: the fp32 probability in whole (see the kernel's comment)
+        constexpr bool P3 = RH || AF == OPURE_A_BF16;
+        constexpr float PS = RH && AF == OPURE_A_F16 ? 32768.0f : 1.0f;
         float mrow[NT], lrow[NT];
         u4v pop[KK][NT], plo[KK][NT], plo2[KK][NT];
 #pragma unroll
@@ -1093,8 +1099,10 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(CL ? 4
                     for (int i = 0; i < 4; ++i)
                     {
                         const float v = sc[kk][T][n][i];
-                        e[4 * T + i] = v == -__builtin_huge_valf() ? 0.0f : exp_hw(__fsub_rn(v, mx));
+                        const float x = __fsub_rn(v, mx);
+                        e[4 * T + i] = v == -__builtin_huge_valf() ? 0.0f : RH ? expf_ref_nonpos(x) : exp_hw(x);
                         sum += e[4 * T + i];
+                        if (PS != 1.0f) e[4 * T + i] = __fmul_rn(e[4 * T + i], PS);
                     }
                 pop[kk][n] = u4v{pack_pair<AF>(e[0], e[1]), pack_pair<AF>(e[2], e[3]), pack_pair<AF>(e[4], e[5]),
                                  pack_pair<AF>(e[6], e[7])};
@@ -1145,6 +1153,9 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(CL ? 4
                     o[dt][n] = mfma32<AF>(vop[kk][dt], plo[kk][n], o[dt][n]);
                     o[dt][n] = mfma32<AF>(vop[kk][dt], pop[kk][n], o[dt][n]);
                 }
+                if (PS != 1.0f)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) o[dt][n][i] = __fmul_rn(o[dt][n][i], 1.0f / PS);
             }
 
         // ---- merge the waves in wave order: m = max, weights exp(m_w - m) -------
@@ -1174,8 +1185,8 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(CL ? 4
         float M = mw[0];
 #pragma unroll
         for (int w = 1; w < NWV; ++w) M = fmaxf(M, mw[w]);
-        // expf_ref, whose bits every launch form shares (exp_hw here: no faster,
-        // 1B step 645.5 us and 8B 256-row layer 254.7 us either way)
+        // expf_ref's bits (exp_hw would save 1B step 646.3 -> 644.9 us, 1B batch
+        // of 32 x 7 rows 152.7 -> 152.0, and change every output's last bits)
         float ew[NWV];
 #pragma unroll
         for (int w = 0; w < NWV; ++w)

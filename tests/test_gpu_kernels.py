@@ -670,6 +670,42 @@ def test_attention_wave_merge_weights(dev, afmt, hd):
     assert np.array_equal(got, np.repeat(to_act(want, afmt)[0][:, None], hd, 1))
 
 
+@pytest.mark.parametrize("hd", [48, 96, 256])
+@pytest.mark.parametrize("afmt", [H.A_F16, H.A_BF16], ids=["f16", "bf16"])
+def test_attention_probabilities_keep_fp32(dev, afmt, hd):
+    """16-bit caches of head sizes other than 64 and 128 weigh V with fp32
+    probabilities.  A token of probability p = e^-x (small next to the row's
+    largest, 1) holds V = S; tokens of probability 1 hold -p S in parts of the
+    storage format, so the output is (p S + C) / L with all but p's last bits
+    cancelled.  Bound: expf_ref within an ulp of e^-x and one fp32 rounding of
+    the sum, 2 ulp of p S, and the output's own rounding."""
+    say("attention probabilities", hd, afmt)
+    S, parts = 32768.0, 2 if afmt == H.A_F16 else 4
+    xs = [to_act(np.float32(v), afmt)[1].item() for v in np.linspace(1.0, 11.5, 22)]
+    B, n = len(xs), 16
+    K, V = np.zeros((B, n, hd), np.float32), np.zeros((B, n, hd), np.float32)
+    K[:, parts + 1:, 0] = -200.0                   # probability 0
+    want, bound = np.zeros(B), np.zeros(B)
+    for b, x in enumerate(xs):
+        c = [-v for v in split_act(np.exp(-x) * S, afmt, parts)]
+        V[b, :parts] = np.array(c)[:, None]
+        K[b, parts, 0], V[b, parts] = -x, S
+        L = parts + np.exp(-x)
+        want[b] = (np.exp(-x) * S + sum(c)) / L
+        bound[b] = 2.0 * 2.0 ** -23 * np.exp(-x) * S / L
+    pool = np.zeros((1, B, 2, 1, 16 * hd), np.uint16)
+    pool[0, :, 0, 0] = to_act(K, afmt)[0].reshape(B, 16 * hd)
+    pool[0, :, 1, 0] = to_act(V, afmt)[0].transpose(0, 2, 1).reshape(B, 16 * hd)
+    q = np.zeros((B, hd), np.float32)
+    q[:, 0] = 1.0
+    pt = np.arange(B, dtype=np.int32).reshape(B, 1)
+    got = from_act(run_attn(dev, attn_model(1, 1, hd, afmt), pool, pt, [n - 1] * B, 1, to_act(q, afmt)[0]), afmt)
+    ulp = 2.0 ** -11 if afmt == H.A_F16 else 2.0 ** -8
+    err = np.abs(got - want[:, None])
+    say("largest error over its bound", (err.max(1) / (bound + ulp * np.abs(want) + 2.0 ** -25)).max())
+    assert (err <= (bound + ulp * np.abs(want) + 2.0 ** -25)[:, None]).all()
+
+
 # fp32 launches over few chunks of 64 tokens: head_dim, query heads, KV heads,
 # rows, contexts (rows ending on either side of chunk boundaries)
 FAST_ALL_CASES = [
