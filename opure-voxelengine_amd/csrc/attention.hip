@@ -1848,6 +1848,21 @@ int attn_prompt_validate(const opure_model* m, const opure_kv* kv, uint32_t rows
     return OPURE_OK;
 }
 
+// k_attn_prompt walks the cache once a workgroup (about 1 us a 64-token tile at
+// head_dim 64, 1.9 at 128), so while its workgroups fill at most half of the
+// CUs a long cache is split over chunks instead: from 16 tokens a workgroup on.
+// A 1B layer's step, unsplit against split: 17 rows (16 workgroups) at 256
+// tokens 50.5 / 50.2 us, 4,096 116 / 58, 15,000 303 / 77; 129 rows (72) at 1,024
+// 105.5 / 100.4, 512 97.7 / 96.0; 256 rows (128) at 2,048 138 / 136, 1,024 121 /
+// 123; 384 rows (192) at 15,000 396 / 479.  8B: 17 rows at 8,000 312 / 100,
+// 256 rows at 2,048 308 / 290.
+bool attn_prompt_splits(const opure_dev* dev, const opure_model* m, uint32_t rows, uint32_t max_ctx)
+{
+    const uint64_t wgs = static_cast<uint64_t>(m->n_kv_heads) * ((static_cast<uint64_t>(rows) * (m->n_heads / m->n_kv_heads) + 63u) / 64u);
+    const uint32_t n_cu = dev && dev->n_cu > 0 ? static_cast<uint32_t>(dev->n_cu) : 256u;
+    return 2u * wgs <= n_cu && max_ctx >= 16u * wgs;
+}
+
 int attn_prompt_launch(opure_dev* dev, const opure_model* m, const opure_kv* kv, uint32_t layer, uint32_t rows,
                        const int32_t* seq_len, uint32_t max_ctx, const void* q, void* out)
 {
@@ -1954,7 +1969,8 @@ int attn_launch(opure_dev* dev, const opure_model* m, const opure_kv* kv, uint32
             // of the partials written and read, a chunk's page-table entries
             // loaded while the chunk before computes, a chunk past a
             // sequence's end costs no round trip of its own
-            const bool fold = hd == 64u && static_cast<uint64_t>(p.n_kv) * p.nch * batch > 8ull * n_cu;
+            const bool prompt = rows > OPURE_MAX_ROWS;
+            const bool fold = hd == 64u && !prompt && static_cast<uint64_t>(p.n_kv) * p.nch * batch > 8ull * n_cu;
             const dim3 fgrid(p.n_kv, (p.nch + ATTN_GROUP - 1u) / ATTN_GROUP, batch);
             if (fold)
             {
@@ -1962,17 +1978,23 @@ int attn_launch(opure_dev* dev, const opure_model* m, const opure_kv* kv, uint32
                 p.cpp = ATTN_GROUP;
                 grp = 1u;
             }
-            // head_dim 128 over more than 32 query rows (a prompt's parts): the
-            // 32-row blocks along z of one launch -- a launch a block ended in a
-            // last wave of workgroups each (640 on 512 slots)
-            if (hd == 128u && Gq > 32u && batch * ((Gq + 31u) / 32u) <= 65535u)
+            // head_dim 128 over more than 32 query rows (a prompt's parts), and
+            // a prompt step's rows: the 32-row blocks along z of one launch -- a
+            // launch a block ended in a last wave of workgroups each (640 on 512
+            // slots)
+            if ((prompt || (hd == 128u && Gq > 32u)) && batch * ((Gq + 31u) / 32u) <= 65535u)
             {
                 AttnParams pq = p;
                 pq.qoff = 0u;
                 pq.zt = (Gq + 31u) / 32u;
                 const dim3 g(p.n_kv, p.nch, batch * pq.zt);
-                const int rc = p.afmt == OPURE_A_F16 ? launch_mfma<128, OPURE_A_F16, 2, 2, 4, true>(dev, g, pq)
-                                                     : launch_mfma<128, OPURE_A_BF16, 2, 2, 4, true>(dev, g, pq);
+                int rc;
+                if (hd == 64u)
+                    rc = p.afmt == OPURE_A_F16 ? launch_mfma<64, OPURE_A_F16, 2, 1, 4, true>(dev, g, pq)
+                                               : launch_mfma<64, OPURE_A_BF16, 2, 1, 4, true>(dev, g, pq);
+                else
+                    rc = p.afmt == OPURE_A_F16 ? launch_mfma<128, OPURE_A_F16, 2, 2, 4, true>(dev, g, pq)
+                                               : launch_mfma<128, OPURE_A_BF16, 2, 2, 4, true>(dev, g, pq);
                 if (rc) return rc;
             }
             else

@@ -252,6 +252,8 @@ uint64_t attn_partial_bytes(uint32_t batch, uint32_t n_kv, uint32_t group, uint3
 int      attn_validate(const opure_model* m, const opure_kv* kv, uint32_t batch, uint32_t rows, uint32_t max_ctx);
 // a prompt's rows of one sequence (16-bit caches, head_dim 64 or 128)
 int      attn_prompt_validate(const opure_model* m, const opure_kv* kv, uint32_t rows, uint32_t max_ctx);
+// whether a prompt step's rows take the split kernels (attn_launch) instead
+bool     attn_prompt_splits(const opure_dev* dev, const opure_model* m, uint32_t rows, uint32_t max_ctx);
 int      attn_prompt_launch(opure_dev* dev, const opure_model* m, const opure_kv* kv, uint32_t layer, uint32_t rows,
                             const int32_t* seq_len, uint32_t max_ctx, const void* q, void* out);
 int      attn_launch(opure_dev* dev, const opure_model* m, const opure_kv* kv, uint32_t layer, uint32_t batch,

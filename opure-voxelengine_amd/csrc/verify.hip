@@ -192,8 +192,9 @@ struct VerifyPlan {
     uint32_t lm_tiles = 0;
 };
 
-// prompt: one sequence's R rows, of which only the last gets (split) attention
-// in the last layer, logits and their argmax
+// prompt: one sequence's R rows, of which only the last gets attention in the
+// last layer (split, as every row's is behind a long cache), logits and their
+// argmax
 static VerifyPlan make_plan(const opure_dev* dev, const opure_model* m, uint32_t B, uint32_t R, uint32_t max_ctx,
                             bool prompt = false)
 {
@@ -215,7 +216,8 @@ static VerifyPlan make_plan(const opure_dev* dev, const opure_model* m, uint32_t
     const uint64_t am = std::max<uint64_t>(p.lm_tiles, argmax_parts(m->vocab)) * (prompt ? 1u : MR) * 4u;
     p.am_val = take(am);
     p.am_idx = take(am);
-    p.attn = take(attn_partial_bytes(B, m->n_kv_heads, m->n_heads / m->n_kv_heads, prompt ? 1u : R, m->head_dim, m->afmt, max_ctx));
+    const uint32_t attn_rows = !prompt || attn_prompt_splits(dev, m, R, max_ctx) ? R : 1u;
+    p.attn = take(attn_partial_bytes(B, m->n_kv_heads, m->n_heads / m->n_kv_heads, attn_rows, m->head_dim, m->afmt, max_ctx));
     p.rej = take(prompt ? 0u : accept_ws_bytes(B, R - 1u, m->vocab, OPURE_ACCEPT_REJECTION));
     // split-K accumulators of the GEMVs over more than OPURE_MAX_ROWS rows
     uint64_t part = 0;
@@ -384,8 +386,9 @@ static int layer_launch(opure_dev* dev, const opure_model* m, const opure_kv* kv
     int rc;
     if ((rc = qkv_launch(dev, m, kv, L, R, seq_len, P, x, ss, c, xn_ready))) return rc;
     if ((rc = prof_begin(dev, OPURE_STAGE_ATTN)) ||
-        (rc = c.prompt ? attn_prompt_launch(dev, m, kv, L, R, seq_len, max_ctx, q, att)
-                       : attn_launch(dev, m, kv, L, B, R, seq_len, max_ctx, q, att, reinterpret_cast<float*>(ws + P.attn))) ||
+        (rc = c.prompt && !attn_prompt_splits(dev, m, R, max_ctx)
+                  ? attn_prompt_launch(dev, m, kv, L, R, seq_len, max_ctx, q, att)
+                  : attn_launch(dev, m, kv, L, B, R, seq_len, max_ctx, q, att, reinterpret_cast<float*>(ws + P.attn))) ||
         (rc = prof_end(dev)))
         return rc;
     return post_attention_launch(dev, m, L, P, x, ss, c, next_gain);

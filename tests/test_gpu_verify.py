@@ -141,6 +141,37 @@ def test_prompt_step_matches_oracle(dev, wfmt, afmt, hd, rows, start):
     assert np.array_equal(pools[0], pools[1])
 
 
+@pytest.mark.parametrize("wfmt,afmt,hd,heads,rows,start", [
+    (O.W_I8PC, O.A_F16, 64, (8, 2), 48, 2103), (O.W_I4G128, O.A_BF16, 64, (16, 4), 240, 1000),
+    (O.W_I4G128, O.A_F16, 128, (16, 2), 96, 517)], ids=lambda v: str(v))
+def test_prompt_step_behind_a_long_cache_same_bits(dev, wfmt, afmt, hd, heads, rows, start):
+    """Few rows behind a long cache take the split attention of the verify step
+    (k_attn_prompt would leave most of the chip idle while it walks the cache):
+    up to 256 rows the prompt step appends, in every layer, the K/V bits of a
+    verify step over the same rows in parts of 16."""
+    say("prompt step, long cache", wfmt, afmt, hd, heads, rows, start)
+    parts = rows // 16
+    m = small_model(wfmt, afmt, n_layers=3, hd=hd, heads=heads, ffn=1024, max_pos=4096, attn_scale=hd ** -0.5, tied=True)
+    cap = (start + rows + 16) // 16 * 16
+    kv = random_cache(m, 1, cap, cap // 16 + 3, seed=rows)
+    tokens = np.random.default_rng(rows).integers(0, m.cfg["vocab"], rows).astype(np.int32)
+    dm = device_model(dev, m)
+    one = device_kv(dev, m, kv)
+    io = dev.upload(np.concatenate([tokens, start + 16 * np.arange(parts, dtype=np.int32)]))
+    a = H.PromptArgs(C.pointer(dm.desc), C.pointer(one.desc), int(io), int(io) + 4 * rows, rows, start + rows, None, None)
+    H.check(H.lib().opure_prompt_step(dev.h, C.byref(a)))
+    dev.sync()
+    wide = H.DeviceKV(dev, m.cfg, kv.n_pages, parts, kv.max_pages)
+    wide.set_pool(kv.pool)
+    wide.set_page_table(np.repeat(kv.page_table, parts, axis=0))
+    v = H.VerifyArgs()
+    v.model, v.kv, v.batch, v.rows, v.max_ctx = C.pointer(dm.desc), C.pointer(wide.desc), parts, 16, start + rows
+    v.tokens, v.seq_len = int(io), int(io) + 4 * rows
+    H.check(H.lib().opure_verify_step(dev.h, C.byref(v)))
+    dev.sync()
+    assert np.array_equal(one.get_pool(), wide.get_pool())
+
+
 def test_prompt_step_refuses(dev):
     """Rows a verify step takes or too many, fp32, another head size, an
     argmax without logits."""
