@@ -542,11 +542,13 @@ int launch_wide_epi_only(opure_dev* dev, const WParams& wp)
         return OPURE_OK;
     };
     constexpr uint32_t KH = WF == OPURE_W_I8PC ? 2u : 1u;
-    // a prompt's step has workgroups enough for two and more a CU: one set of
-    // waves a workgroup, each wave four weight tiles
-    if (wp.prompt && wp.cgs <= 4u) return go(WideShape<4, 2, 2, 1>{});
+    // an int8 prompt's step: one set of waves a workgroup, each wave four weight
+    // tiles by four column tiles, or two in column groups of half the size
     if constexpr (WF == OPURE_W_I8PC)
+    {
+        if (wp.prompt && wp.cgs <= 4u) return go(WideShape<4, 2, 2, 1>{});
         if (wp.prompt) return go(WideShape<4, 4, 2, 1>{});
+    }
     if (wp.cgs <= 2u) return go(WideShape<1, 2, 1, KH>{});
     if (wp.cgs <= 4u) return go(WideShape<1, 4, 1, KH>{});
     return go(WideShape<2, 8, 1, KH>{});

@@ -258,12 +258,16 @@ WidePlan wide_plan(const opure_dev* dev, uint32_t wfmt, uint32_t out, uint32_t i
     w.nrg = (w.tiles + WIDE_RT - 1u) / WIDE_RT;
     const uint32_t cus = dev && dev->n_cu > 0 ? static_cast<uint32_t>(dev->n_cu) : 256u;
     w.ncg = (w.mt + WIDE_CG - 1u) / WIDE_CG;
-    // a prompt's step with one to two workgroups a CU: column groups of half
-    // the size (1B qkv over 1,436 rows: 288 workgroups -> 552, 54 -> 47 us).
-    // Fewer workgroups are split over K instead (o_proj and down, 192: 36 and
-    // 87 us with the next rmsnorm, 37 and 109 in halves).
+    // an int8 prompt's step with between one and two workgroups a CU: column
+    // groups of half the size (1B qkv over 1,436 rows: 288 workgroups -> 552,
+    // 54 -> 47 us; a layer's step at 257 rows 132 -> 128 us, at 1,900 403 ->
+    // 395).  One workgroup on every CU stays (o_proj and down at 2,048 rows:
+    // 425 us a layer, 433 in halves); fewer are split over K instead (o_proj and
+    // down, 192: 36 and 87 us with the next rmsnorm, 37 and 109 in halves).
+    // uint4's decode of a weight tile is shared by half as many columns then:
+    // an 8B layer's step at 1,200 rows 895 us, 975 in halves, at 1,900 1,230 / 1,360.
     const uint32_t wgs = w.nrg * w.ncg;
-    if (M > OPURE_MAX_BATCH_ROWS && wgs >= cus && wgs < 2u * cus) w.ncg = (w.mt + WIDE_CG / 2u - 1u) / (WIDE_CG / 2u);
+    if (M > OPURE_MAX_BATCH_ROWS && wfmt == OPURE_W_I8PC && wgs > cus && wgs < 2u * cus) w.ncg = (w.mt + WIDE_CG / 2u - 1u) / (WIDE_CG / 2u);
     w.cgs = (w.mt + w.ncg - 1u) / w.ncg;
     // split K while there are fewer row groups than half the CUs (a batch
     // over 128 rows has two column groups), at most 8 ways and U blocks a split

@@ -99,18 +99,13 @@ def test_layer_norm_rows_same_bits(dev, hidden, afmt):
     assert np.array_equal(pools[0], pools[1]) and not np.array_equal(pools[0], kv.pool)
 
 
-@pytest.mark.parametrize("rows,start", [(17, 0), (33, 100), (130, 37), (300, 37), (777, 0)])
-@pytest.mark.parametrize("wfmt,afmt,hd", [(O.W_I8PC, O.A_F16, 64), (O.W_I4G128, O.A_F16, 128), (O.W_I4G128, O.A_BF16, 64)],
-                         ids=["i8-f16-hd64", "i4-f16-hd128", "i4-bf16-hd64"])
-def test_prompt_step_matches_oracle(dev, wfmt, afmt, hd, rows, start):
-    """A prompt of one sequence behind `start` cached positions (a page's
-    middle), up to a batch's rows and past them, with and without K splits:
-    the appended K/V of both layers, the last row's logits and their argmax
-    against the oracle's row by row, within the bars above (bf16: one storage
-    ulp more on K/V, whose values reach past 4); without logits the same K/V."""
-    say("prompt step", wfmt, afmt, hd, rows, start)
+def check_prompt_step(dev, m, rows, start):
+    """One prompt step of `rows` tokens behind `start` cached positions: the
+    appended K/V of every layer, the last row's logits and their argmax against
+    the oracle's row by row, within the bars above (bf16: one storage ulp more
+    on K/V, whose values reach past 4); without logits the same K/V."""
     import npref
-    m = small_model(wfmt, afmt, hd=hd, ffn=2048, attn_scale=hd ** -0.5, tied=wfmt != O.W_I4G128)
+    afmt = m.cfg["afmt"]
     cap = (start + rows + 16) // 16 * 16
     kv = random_cache(m, 1, cap, cap // 16 + 3, seed=rows)
     tokens = np.random.default_rng(rows).integers(0, m.cfg["vocab"], (1, rows)).astype(np.int32)
@@ -139,6 +134,35 @@ def test_prompt_step_matches_oracle(dev, wfmt, afmt, hd, rows, start):
     g, w = npref.act_to_f32(pools[0], afmt), npref.act_to_f32(kv_o.pool, afmt)
     assert (np.abs(g - w) <= 2e-2 + (2.0 ** -7 * np.abs(w) if afmt == O.A_BF16 else 0.0)).all()
     assert np.array_equal(pools[0], pools[1])
+
+
+@pytest.mark.parametrize("rows,start", [(17, 0), (33, 100), (130, 37), (300, 37), (777, 0)])
+@pytest.mark.parametrize("wfmt,afmt,hd", [(O.W_I8PC, O.A_F16, 64), (O.W_I4G128, O.A_F16, 128), (O.W_I4G128, O.A_BF16, 64)],
+                         ids=["i8-f16-hd64", "i4-f16-hd128", "i4-bf16-hd64"])
+def test_prompt_step_matches_oracle(dev, wfmt, afmt, hd, rows, start):
+    """A prompt of one sequence behind `start` cached positions (a page's
+    middle), up to a batch's rows and past them, with and without K splits:
+    the appended K/V of both layers, the last row's logits and their argmax
+    against the oracle's row by row, within the bars above (bf16: one storage
+    ulp more on K/V, whose values reach past 4); without logits the same K/V."""
+    say("prompt step", wfmt, afmt, hd, rows, start)
+    m = small_model(wfmt, afmt, hd=hd, ffn=2048, attn_scale=hd ** -0.5, tied=wfmt != O.W_I4G128)
+    check_prompt_step(dev, m, rows, start)
+
+
+@pytest.mark.parametrize("rows,hidden,heads,ffn", [(1437, 256, (32, 8), 2048), (1437, 2816, (4, 2), 512),
+                                                   (257, 256, (4, 2), 8192), (2048, 512, (16, 8), 512)], ids=lambda v: str(v))
+@pytest.mark.parametrize("wfmt,afmt,hd", [(O.W_I8PC, O.A_F16, 64), (O.W_I4G128, O.A_F16, 64), (O.W_I4G128, O.A_BF16, 64)],
+                         ids=["i8-f16", "i4-f16", "i4-bf16"])
+def test_prompt_step_gemm_shapes_match_oracle(dev, wfmt, afmt, hd, rows, hidden, heads, ffn):
+    """Sizes at which a GEMM of the prompt step has between one and two
+    workgroups a CU (int8 halves its column groups): QKV and gate/up (288 and
+    384 workgroups), the residual ones (264), gate/up at the fewest rows past a
+    batch's (384); and the most rows of a step."""
+    say("prompt step shapes", wfmt, afmt, rows, hidden, heads, ffn)
+    m = small_model(wfmt, afmt, hd=hd, hidden=hidden, heads=heads, ffn=ffn, attn_scale=hd ** -0.5, max_pos=2048,
+                    tied=wfmt != O.W_I4G128)
+    check_prompt_step(dev, m, rows, 0)
 
 
 @pytest.mark.parametrize("wfmt,afmt,hd,heads,rows,start", [
