@@ -1283,7 +1283,7 @@ __global__ __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(CL ? 4
 
 // Attention of a prompt's rows of one sequence (16-bit caches, head_dim 64 or
 // 128): a workgroup takes 64 NT query rows of a KV head (row qi = j group + head,
-// 16 NT a wave; NT 2 once that leaves several workgroups a CU) over tiles of 64 tokens, keeping each row's running maximum, sum
+// 16 NT a wave) over tiles of 64 tokens, keeping each row's running maximum, sum
 // and output in registers, so nothing is split, merged or read twice: the
 // split kernel above reads the cache once per 16 positions and writes
 // partials for a combine (1,437 tokens of the 1B shape 230 us a layer, 43
@@ -1883,9 +1883,13 @@ int attn_prompt_launch(opure_dev* dev, const opure_model* m, const opure_kv* kv,
     p.scale = m->attn_scale;
     p.err = dev->err;
     const uint32_t Gq = rows * (p.n_heads / p.n_kv), n_cu = dev->n_cu > 0 ? static_cast<uint32_t>(dev->n_cu) : 256u;
-    // 128 rows a workgroup read each tile from LDS for twice the work, once
-    // there are four such workgroups a CU to overlap; below, 64
-    const bool two = static_cast<uint64_t>(p.n_kv) * ((Gq + 127u) / 128u) >= 4ull * n_cu;
+    // 128 rows a workgroup read each tile from LDS for twice the work: with four
+    // such workgroups a CU to overlap (64 heads and 2,048 rows), behind a cache
+    // at least as long as the prompt.  A step of 4 layers, 64 rows a workgroup
+    // against 128: 64 heads of 128 at start 2,048 2,735 / 2,530 us, 10,000 6,170 /
+    // 5,381; of 64 at 2,048 1,820 / 1,791; from position 0, where the causal rows of
+    // a workgroup see fewer tiles than its last, 1,784 / 1,803 and 1,236 / 1,270
+    const bool two = static_cast<uint64_t>(p.n_kv) * ((Gq + 127u) / 128u) >= 4ull * n_cu && max_ctx >= 2u * rows;
     const dim3 grid(p.n_kv, two ? (Gq + 127u) / 128u : (Gq + 63u) / 64u);
     auto go = [&](auto one, auto pair) { OPURE_LAUNCH(dev, (two ? pair : one), grid, dim3(256), 0, p); };
     const bool h = m->afmt == OPURE_A_F16;

@@ -196,6 +196,37 @@ def test_prompt_step_behind_a_long_cache_same_bits(dev, wfmt, afmt, hd, heads, r
     assert np.array_equal(one.get_pool(), wide.get_pool())
 
 
+@pytest.mark.parametrize("wfmt,afmt,hd", [(O.W_I8PC, O.A_F16, 64), (O.W_I4G128, O.A_BF16, 64), (O.W_I4G128, O.A_F16, 128),
+                                          (O.W_I4G128, O.A_BF16, 128)], ids=["i8-f16-64", "i4-bf16-64", "i4-f16-128", "i4-bf16-128"])
+def test_prompt_step_row_blocks_agree(dev, wfmt, afmt, hd):
+    """64 heads and 2,041 rows behind 2,050 cached positions take 128 query rows a
+    workgroup (the last one ragged); the same rows in two steps take 64.  Tiles
+    start at multiples of 64 from position 0 either way, so the rows of the
+    second layer's K/V agree within the bars above (their GEMMs may sum in
+    another order)."""
+    import npref
+    say("prompt step row blocks", wfmt, afmt, hd)
+    rows, start, half = 2041, 2050, 1021
+    m = small_model(wfmt, afmt, hd=hd, heads=(64, 8), hidden=256, ffn=512, attn_scale=hd ** -0.5, max_pos=4096, tied=True)
+    cap = 4096
+    kv = random_cache(m, 1, cap, cap // 16 + 3, seed=hd)
+    tokens = np.random.default_rng(hd).integers(0, m.cfg["vocab"], rows).astype(np.int32)
+    dm = device_model(dev, m)
+    io = dev.upload(np.concatenate([tokens, np.array([start, start + half], np.int32)]))
+    pools = []
+    for parts in ([(0, rows)], [(0, half), (half, rows)]):
+        dkv = device_kv(dev, m, kv)
+        for i, (a0, a1) in enumerate(parts):
+            a = H.PromptArgs(C.pointer(dm.desc), C.pointer(dkv.desc), int(io) + 4 * a0, int(io) + 4 * (rows + i), a1 - a0,
+                             start + a1, None, None)
+            H.check(H.lib().opure_prompt_step(dev.h, C.byref(a)))
+        dev.sync()
+        pools.append(npref.act_to_f32(dkv.get_pool(), afmt))
+    g, w = pools
+    assert np.isfinite(g).all() and not np.array_equal(g[1], npref.act_to_f32(kv.pool, afmt)[1])
+    assert (np.abs(g - w) <= 2e-2 + (2.0 ** -7 * np.abs(w) if afmt == O.A_BF16 else 0.0)).all()
+
+
 def test_prompt_step_refuses(dev):
     """Rows a verify step takes or too many, fp32, another head size, an
     argmax without logits."""
