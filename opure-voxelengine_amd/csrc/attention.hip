@@ -1716,14 +1716,17 @@ int launch_mfma(opure_dev* dev, dim3 grid, const AttnParams& p)
 }
 
 // A 16-bit cache of any other head size, on matrix cores: 128-token chunks
-// (4 waves x 32 tokens), every block of query rows in one launch.  Two
-// 16-row blocks a workgroup up to head_dim 128; past that the output tiles of
-// a second block do not fit beside the K and V operands, so one.
+// (4 waves x 32 tokens), every block of query rows in one launch.  Up to 16
+// query rows are one block a workgroup (a second one would be computed for
+// nothing: 32 sequences of 5 rows, 3,000 tokens, heads of 80 63 us with it, 47
+// without; 1 x 1 row of 96 10.3 / 9.2).  More are two up to head_dim 128; past
+// that the output tiles of a second block do not fit beside the K and V
+// operands.
 template <int HDP, int AF>
 int launch_mfma_hd(opure_dev* dev, AttnParams p, uint32_t Gq, uint32_t batch)
 {
     constexpr int NT2 = HDP <= 128 ? 2 : 1;
-    if (HDP > 32 && HDP % 64 == 0 && Gq <= 16u)
+    if (Gq <= 16u)
     {
         p.zt = 1u;
         return launch_mfma<HDP, AF, 1, 1, 4, true, false, true>(dev, dim3(p.n_kv, p.nch, batch), p);
