@@ -171,7 +171,7 @@ __global__ __launch_bounds__(256) void k_attn_chunk_generic(AttnParams p)
     }
 }
 
-// Fast path for head_dim <= 128 and 64-token chunks.  The chunk's K and V
+// fp32 fast path for head_dim 64 and 128, 64-token chunks.  The chunk's K and V
 // slices of this KV head are staged once in LDS with 128-bit loads; each wave
 // then keeps one K row per lane (lane = token) and one or two V columns per
 // lane (lane = channel) in registers and walks its share of the query rows:
@@ -199,11 +199,11 @@ constexpr uint32_t attn_fast_threads()
     return HD == 64 ? 512u : 256u;
 }
 
-template <int HD, int AF, bool ALL>
+template <int HD, bool ALL>
 __global__ __launch_bounds__(attn_fast_threads<HD>()) void k_attn_chunk(AttnParams p)
 {
     constexpr uint32_t NT = attn_fast_threads<HD>(), NWV = NT / 64u, RB = 2;   // RB: rows a wave scores together
-    constexpr uint32_t CH = 64, EB = AF == OPURE_A_F32 ? 4u : 2u, PPC = CH / OPURE_PAGE_SIZE;
+    constexpr uint32_t CH = 64, EB = 4, PPC = CH / OPURE_PAGE_SIZE;
     constexpr uint32_t ROWB = HD * EB + 16u;              // padded LDS row (bank spread)
     constexpr uint32_t DPL = (HD + 63u) / 64u;             // V channels per lane
     constexpr uint32_t VROWB = CH * EB + 16u;              // padded LDS V column (channel-major)
@@ -236,7 +236,7 @@ __global__ __launch_bounds__(attn_fast_threads<HD>()) void k_attn_chunk(AttnPara
         for (uint32_t u = 0; u < QU; ++u)
         {
             const uint32_t e = e0 + threadIdx.x + NT * u, j = e / GH;
-            qv[u] = e < Gq * HD ? load_act_rt(p.q, (static_cast<uint64_t>(b * R + j) * p.n_heads + kh * group) * HD + (e - j * GH), AF)
+            qv[u] = e < Gq * HD ? static_cast<const float*>(p.q)[(static_cast<uint64_t>(b * R + j) * p.n_heads + kh * group) * HD + (e - j * GH)]
                                 : 0.0f;
         }
     };
@@ -271,7 +271,7 @@ __global__ __launch_bounds__(attn_fast_threads<HD>()) void k_attn_chunk(AttnPara
     constexpr uint32_t TPP = 16u / EB;                     // tokens per V piece
     constexpr uint32_t NPC = (CH * KP + HD * VP) / NT;     // pieces a thread stages a chunk
     static_assert((CH * KP) % NT == 0 && (HD * VP) % NT == 0, "K and V pieces split evenly over the threads");
-    const uint32_t nan = AF == OPURE_A_F32 ? 0x7FC00000u : (AF == OPURE_A_F16 ? 0x7E007E00u : 0x7FC07FC0u);
+    const uint32_t nan = 0x7FC00000u;
     u4v buf[NPC];
     uint32_t tail = 0u;                                    // pieces whose slots past the cache read 0
     auto piece = [&](uint32_t k, bool& isk, uint32_t& row, uint32_t& pc) {
@@ -321,7 +321,7 @@ __global__ __launch_bounds__(attn_fast_threads<HD>()) void k_attn_chunk(AttnPara
             uint32_t row, pc;
             piece(k, isk, row, pc);
             u4v val = buf[k];
-            if (tail & (1u << k)) val = mask_tail<AF>(val, total - (c * CH + pc * TPP));   // slots past the cache read 0
+            if (tail & (1u << k)) val = mask_tail<OPURE_A_F32>(val, total - (c * CH + pc * TPP));   // slots past the cache read 0
             if (isk) *reinterpret_cast<u4v*>(kt + row * ROWB + pc * 16u) = val;
             else *reinterpret_cast<u4v*>(vt + row * VROWB + pc * 16u) = val;
         }
@@ -338,12 +338,7 @@ __global__ __launch_bounds__(attn_fast_threads<HD>()) void k_attn_chunk(AttnPara
         // this lane's K row (token t0 + lane) and V channels (lane, lane + 64)
         float kr[HD];
 #pragma unroll
-        for (uint32_t d = 0; d < HD; ++d)
-        {
-            if constexpr (AF == OPURE_A_F32) kr[d] = reinterpret_cast<const float*>(kt + lane * ROWB)[d];
-            else kr[d] = AF == OPURE_A_F16 ? f16_to_f32(reinterpret_cast<const uint16_t*>(kt + lane * ROWB)[d])
-                                           : bf16_to_f32(reinterpret_cast<const uint16_t*>(kt + lane * ROWB)[d]);
-        }
+        for (uint32_t d = 0; d < HD; ++d) kr[d] = reinterpret_cast<const float*>(kt + lane * ROWB)[d];
         float vc[DPL][CH];
 #pragma unroll
         for (uint32_t i = 0; i < DPL; ++i)
@@ -351,7 +346,7 @@ __global__ __launch_bounds__(attn_fast_threads<HD>()) void k_attn_chunk(AttnPara
             const uint32_t d = lane + 64u * i;
 #pragma unroll
             for (uint32_t t = 0; t < CH; ++t)
-                vc[i][t] = d < HD ? load_act_rt(vt + d * VROWB, t, AF) : 0.0f;
+                vc[i][t] = d < HD ? reinterpret_cast<const float*>(vt + d * VROWB)[t] : 0.0f;
         }
         const uint64_t pbase = ((static_cast<uint64_t>(b) * p.n_kv + kh) * p.npart + c) * Gq;
         const uint32_t pos = t0 + lane;
@@ -469,15 +464,14 @@ __global__ __launch_bounds__(attn_fast_threads<HD>()) void k_attn_chunk(AttnPara
                     num = in ? __fmaf_rn(w, v, num) : num;
                 }
                 if (d < HD)
-                    store_act_rt(p.out, (static_cast<uint64_t>(b * R + j) * p.n_heads + head) * HD + d,
-                                 __fdiv_rn(num, dd), p.afmt);
+                    static_cast<float*>(p.out)[(static_cast<uint64_t>(b * R + j) * p.n_heads + head) * HD + d] = __fdiv_rn(num, dd);
             }
             __builtin_amdgcn_wave_barrier();
         }
     }
 }
 
-// Head_dim 64 over at most ATTN_SPLIT_CHUNKS chunks of 64 tokens (a short
+// fp32, head_dim 64 over at most ATTN_SPLIT_CHUNKS chunks of 64 tokens (a short
 // context): a workgroup per (KV head, pair of query rows, sequence) with a
 // wave per chunk, so a batch of one sequence still spreads over many CUs.  A
 // wave loads its chunk's K rows (lane = token) and V columns (lane = channel)
@@ -489,11 +483,11 @@ __global__ __launch_bounds__(attn_fast_threads<HD>()) void k_attn_chunk(AttnPara
 constexpr uint32_t ATTN_SPLIT_CHUNKS = 8;
 constexpr uint32_t attn_split_lds(uint32_t chunks) { return chunks * 64u * (64u * 4u + 16u); }
 
-template <int AF, bool TURN>
+template <bool TURN>
 __global__ __launch_bounds__(64 * ATTN_SPLIT_CHUNKS) void k_attn_split(AttnParams p)
 {
     constexpr uint32_t HD = 64, CH = 64, RB = 2, NW = ATTN_SPLIT_CHUNKS, PPC = CH / OPURE_PAGE_SIZE;
-    constexpr uint32_t EB = AF == OPURE_A_F32 ? 4u : 2u, EPP = 16u / EB;   // elements a 16-byte piece
+    constexpr uint32_t EB = 4, EPP = 16u / EB;             // elements a 16-byte piece
     __shared__ __align__(16) float qsm[NW][RB][HD];       // each wave's copy of the pair's Q rows
     __shared__ __align__(16) float pbuf[NW][RB][CH];
     __shared__ __align__(16) float pa[NW][RB][HD];        // the chunks' outputs
@@ -519,7 +513,7 @@ __global__ __launch_bounds__(64 * ATTN_SPLIT_CHUNKS) void k_attn_split(AttnParam
         qi[r] = has[r] ? q0 + r : q0;
         jr[r] = qi[r] / group;
         const uint32_t head = kh * group + (qi[r] - jr[r] * group);
-        qv[r] = load_act_rt(p.q, (static_cast<uint64_t>(b * R + jr[r]) * p.n_heads + head) * HD + lane, AF);
+        qv[r] = static_cast<const float*>(p.q)[(static_cast<uint64_t>(b * R + jr[r]) * p.n_heads + head) * HD + lane];
     }
     const uint32_t pi = c * PPC + (lane & (PPC - 1u));
     const int32_t pe = pi < p.max_pages ? pt[pi] : -1;
@@ -541,7 +535,6 @@ __global__ __launch_bounds__(64 * ATTN_SPLIT_CHUNKS) void k_attn_split(AttnParam
         auto safe = [&](int32_t pg_) { return ok(pg_) ? static_cast<uint32_t>(pg_) : 0u; };
         const uint32_t pos = t0 + lane, sl = lane / OPURE_PAGE_SIZE;
         const int32_t kpg = sl == 0u ? pg[0] : sl == 1u ? pg[1] : sl == 2u ? pg[2] : pg[3];
-        static_assert(AF == OPURE_A_F32, "pieces of four values");
         u4v kw[HD / EPP], vw[PPC][OPURE_PAGE_SIZE / EPP];
         if constexpr (!TURN)
         {
@@ -562,56 +555,56 @@ __global__ __launch_bounds__(64 * ATTN_SPLIT_CHUNKS) void k_attn_split(AttnParam
         }
         else
         {
-        constexpr uint32_t ROW = HD * EB + 16u, PLN = OPURE_PAGE_SIZE * HD * EB / 1024u;   // LDS row bytes; loads a plane
-        uint8_t* tl = tile_lds + c * CH * ROW;
-        u4v kraw[PPC][PLN], vraw[PPC][PLN];
+            constexpr uint32_t ROW = HD * EB + 16u, PLN = OPURE_PAGE_SIZE * HD * EB / 1024u;   // LDS row bytes; loads a plane
+            uint8_t* tl = tile_lds + c * CH * ROW;
+            u4v kraw[PPC][PLN], vraw[PPC][PLN];
 #pragma unroll
-        for (uint32_t i = 0; i < PPC; ++i)
-        {
-            const uint8_t* kp = static_cast<const uint8_t*>(p.pool) + kv_elem(p.layer, p.n_pages, safe(pg[i]), 0u, p.n_kv, kh, HD, 0u, 0u) * EB;
-            const uint8_t* vp = static_cast<const uint8_t*>(p.pool) + kv_elem(p.layer, p.n_pages, safe(pg[i]), 1u, p.n_kv, kh, HD, 0u, 0u) * EB;
-#pragma unroll
-            for (uint32_t k = 0; k < PLN; ++k)
+            for (uint32_t i = 0; i < PPC; ++i)
             {
-                kraw[i][k] = *reinterpret_cast<const u4v*>(kp + (k * 64u + lane) * 16u);
-                vraw[i][k] = *reinterpret_cast<const u4v*>(vp + (k * 64u + lane) * 16u);
+                const uint8_t* kp = static_cast<const uint8_t*>(p.pool) + kv_elem(p.layer, p.n_pages, safe(pg[i]), 0u, p.n_kv, kh, HD, 0u, 0u) * EB;
+                const uint8_t* vp = static_cast<const uint8_t*>(p.pool) + kv_elem(p.layer, p.n_pages, safe(pg[i]), 1u, p.n_kv, kh, HD, 0u, 0u) * EB;
+#pragma unroll
+                for (uint32_t k = 0; k < PLN; ++k)
+                {
+                    kraw[i][k] = *reinterpret_cast<const u4v*>(kp + (k * 64u + lane) * 16u);
+                    vraw[i][k] = *reinterpret_cast<const u4v*>(vp + (k * 64u + lane) * 16u);
+                }
             }
-        }
-        auto wave_sync = [] {
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        };
+            auto wave_sync = [] {
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            };
 #pragma unroll
-        for (uint32_t i = 0; i < PPC; ++i)
+            for (uint32_t i = 0; i < PPC; ++i)
 #pragma unroll
-            for (uint32_t k = 0; k < PLN; ++k)
-            {
-                const uint32_t e = k * 64u + lane;                     // piece of the plane: token e / 16
-                *reinterpret_cast<u4v*>(tl + (OPURE_PAGE_SIZE * i + e / (HD / EPP)) * ROW + (e % (HD / EPP)) * 16u) = kraw[i][k];
-            }
-        wave_sync();
+                for (uint32_t k = 0; k < PLN; ++k)
+                {
+                    const uint32_t e = k * 64u + lane;                     // piece of the plane: token e / 16
+                    *reinterpret_cast<u4v*>(tl + (OPURE_PAGE_SIZE * i + e / (HD / EPP)) * ROW + (e % (HD / EPP)) * 16u) = kraw[i][k];
+                }
+            wave_sync();
 #pragma unroll
-        for (uint32_t k = 0; k < HD / EPP; ++k) kw[k] = *reinterpret_cast<const u4v*>(tl + lane * ROW + k * 16u);
-        wave_sync();
+            for (uint32_t k = 0; k < HD / EPP; ++k) kw[k] = *reinterpret_cast<const u4v*>(tl + lane * ROW + k * 16u);
+            wave_sync();
 #pragma unroll
-        for (uint32_t i = 0; i < PPC; ++i)
+            for (uint32_t i = 0; i < PPC; ++i)
 #pragma unroll
-            for (uint32_t k = 0; k < PLN; ++k)
-            {
-                const uint32_t e = k * 64u + lane;                     // channel e / 4, four tokens
-                *reinterpret_cast<u4v*>(tl + (e / 4u) * ROW + OPURE_PAGE_SIZE * EB * i + (e % 4u) * 16u) = vraw[i][k];
-            }
-        wave_sync();
+                for (uint32_t k = 0; k < PLN; ++k)
+                {
+                    const uint32_t e = k * 64u + lane;                     // channel e / 4, four tokens
+                    *reinterpret_cast<u4v*>(tl + (e / 4u) * ROW + OPURE_PAGE_SIZE * EB * i + (e % 4u) * 16u) = vraw[i][k];
+                }
+            wave_sync();
 #pragma unroll
-        for (uint32_t i = 0; i < PPC; ++i)
+            for (uint32_t i = 0; i < PPC; ++i)
 #pragma unroll
-            for (uint32_t k = 0; k < OPURE_PAGE_SIZE / EPP; ++k)
-                vw[i][k] = *reinterpret_cast<const u4v*>(tl + lane * ROW + OPURE_PAGE_SIZE * EB * i + k * 16u);
+                for (uint32_t k = 0; k < OPURE_PAGE_SIZE / EPP; ++k)
+                    vw[i][k] = *reinterpret_cast<const u4v*>(tl + lane * ROW + OPURE_PAGE_SIZE * EB * i + k * 16u);
         }
         // the fills: a position past the cache reads 0, a missing page (or an
         // entry past the table) NaN, a V piece reaching past the cache keeps
         // its slots before the end
-        const uint32_t nan = AF == OPURE_A_F32 ? 0x7FC00000u : (AF == OPURE_A_F16 ? 0x7E007E00u : 0x7FC07FC0u);
+        const uint32_t nan = 0x7FC00000u;
         const u4v zero = {0u, 0u, 0u, 0u}, nanv = {nan, nan, nan, nan};
 #pragma unroll
         for (uint32_t k = 0; k < HD / EPP; ++k) kw[k] = pos < total ? (ok(kpg) ? kw[k] : nanv) : zero;
@@ -621,32 +614,17 @@ __global__ __launch_bounds__(64 * ATTN_SPLIT_CHUNKS) void k_attn_split(AttnParam
             for (uint32_t k = 0; k < OPURE_PAGE_SIZE / EPP; ++k)
             {
                 const uint32_t pp = t0 + i * OPURE_PAGE_SIZE + k * EPP;
-                u4v v = ok(pg[i]) ? (pp + EPP > total ? mask_tail<AF>(vw[i][k], total - pp) : vw[i][k]) : nanv;
+                u4v v = ok(pg[i]) ? (pp + EPP > total ? mask_tail<OPURE_A_F32>(vw[i][k], total - pp) : vw[i][k]) : nanv;
                 vw[i][k] = pp < total ? v : zero;
             }
         float kr[HD], vc[CH];
 #pragma unroll
-        for (uint32_t d = 0; d < HD; ++d)
-        {
-            const uint32_t w = kw[d / EPP][(d % EPP) * EB / 4u];
-            if constexpr (AF == OPURE_A_F32) kr[d] = __uint_as_float(w);
-            else
-            {
-                const uint16_t h = static_cast<uint16_t>(d % 2u ? w >> 16 : w & 0xFFFFu);
-                kr[d] = AF == OPURE_A_F16 ? f16_to_f32(h) : bf16_to_f32(h);
-            }
-        }
+        for (uint32_t d = 0; d < HD; ++d) kr[d] = __uint_as_float(kw[d / EPP][d % EPP]);
 #pragma unroll
         for (uint32_t t = 0; t < CH; ++t)
         {
             const uint32_t i = t / OPURE_PAGE_SIZE, s = t % OPURE_PAGE_SIZE;
-            const uint32_t w = vw[i][s / EPP][(s % EPP) * EB / 4u];
-            if constexpr (AF == OPURE_A_F32) vc[t] = __uint_as_float(w);
-            else
-            {
-                const uint16_t h = static_cast<uint16_t>(s % 2u ? w >> 16 : w & 0xFFFFu);
-                vc[t] = AF == OPURE_A_F16 ? f16_to_f32(h) : bf16_to_f32(h);
-            }
+            vc[t] = __uint_as_float(vw[i][s / EPP][s % EPP]);
         }
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -724,8 +702,7 @@ __global__ __launch_bounds__(64 * ATTN_SPLIT_CHUNKS) void k_attn_split(AttnParam
             num = in ? __fmaf_rn(wsh[r][in ? cc : 0u], pa[in ? cc : 0u][r][lane], num) : num;
         }
         const uint32_t head = kh * group + (qi[r] - jr[r] * group);
-        store_act_rt(p.out, (static_cast<uint64_t>(b * R + jr[r]) * p.n_heads + head) * HD + lane, __fdiv_rn(num, dd),
-                     p.afmt);
+        static_cast<float*>(p.out)[(static_cast<uint64_t>(b * R + jr[r]) * p.n_heads + head) * HD + lane] = __fdiv_rn(num, dd);
     }
 }
 
@@ -1751,17 +1728,17 @@ int launch_mfma_any(opure_dev* dev, const AttnParams& p, uint32_t Gq, uint32_t b
     }
 }
 
-template <int HD, int AF, bool ALL>
+template <int HD, bool ALL>
 int launch_fast(opure_dev* dev, dim3 grid, uint32_t lds, const AttnParams& p)
 {
     static bool configured = false;
     if (!configured)
     {
-        OPURE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_attn_chunk<HD, AF, ALL>),
+        OPURE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_attn_chunk<HD, ALL>),
                                           hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024));
         configured = true;
     }
-    OPURE_LAUNCH(dev, (k_attn_chunk<HD, AF, ALL>), grid, dim3(attn_fast_threads<HD>()), lds, p);
+    OPURE_LAUNCH(dev, (k_attn_chunk<HD, ALL>), grid, dim3(attn_fast_threads<HD>()), lds, p);
     OPURE_LAUNCH_CHECK("k_attn_chunk");
     return OPURE_OK;
 }
@@ -2046,14 +2023,14 @@ int attn_launch(opure_dev* dev, const opure_model* m, const opure_kv* kv, uint32
             static bool configured = false;
             if (!configured)
             {
-                OPURE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_attn_split<OPURE_A_F32, true>),
+                OPURE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_attn_split<true>),
                                                   hipFuncAttributeMaxDynamicSharedMemorySize,
                                                   static_cast<int>(attn_split_lds(ATTN_SPLIT_CHUNKS))));
                 configured = true;
             }
-            OPURE_LAUNCH(dev, (k_attn_split<OPURE_A_F32, true>), g, blk, attn_split_lds(p.nch), p);
+            OPURE_LAUNCH(dev, (k_attn_split<true>), g, blk, attn_split_lds(p.nch), p);
         }
-        else OPURE_LAUNCH(dev, (k_attn_split<OPURE_A_F32, false>), g, blk, 0, p);
+        else OPURE_LAUNCH(dev, (k_attn_split<false>), g, blk, 0, p);
         OPURE_LAUNCH_CHECK("k_attn_split");
         return OPURE_OK;
     }
@@ -2066,8 +2043,8 @@ int attn_launch(opure_dev* dev, const opure_model* m, const opure_kv* kv, uint32
         const uint32_t lds = all ? static_cast<uint32_t>(all_lds) : Gq * hd * 4u;
         const dim3 g = all ? dim3(p.n_kv, 1u, batch) : grid;
         int rc;
-        if (hd == 64u) rc = launch_fast<64, OPURE_A_F32, false>(dev, g, lds, p);
-        else rc = all ? launch_fast<128, OPURE_A_F32, true>(dev, g, lds, p) : launch_fast<128, OPURE_A_F32, false>(dev, g, lds, p);
+        if (hd == 64u) rc = launch_fast<64, false>(dev, g, lds, p);
+        else rc = all ? launch_fast<128, true>(dev, g, lds, p) : launch_fast<128, false>(dev, g, lds, p);
         if (rc) return rc;
         if (all) return OPURE_OK;
     }
