@@ -181,14 +181,15 @@ def test_verify_step_and_rollback_kv_c1(models):
     eng.close()
 
 
-def test_prefill_256_rows_engine():
-    """A quantised model's 300-token prompt is prefilled 256 rows a launch
-    (16 parts x 16 rows on one page-table row), then 32, then 11 in a 16-row
-    step: the greedy continuation equals the oracle's (every decision's top-2
-    gap is well above the logit bar)."""
+@pytest.mark.parametrize("hd", [64, 96], ids=["prompt-step", "256-rows"])
+def test_prefill_256_rows_engine(hd):
+    """A quantised model's 300-token prompt: at head_dim 64 one prompt step, at
+    96 256 rows a launch (16 parts x 16 rows on one page-table row), then 32,
+    then 11 in a 16-row step.  The greedy continuation equals the oracle's
+    (every decision's top-2 gap is well above the logit bar)."""
     from test_gpu_verify import small_model
     from gpu_util import device_model
-    m = small_model(O.W_I8PC, O.A_F16, max_pos=512)
+    m = small_model(O.W_I8PC, O.A_F16, hd=hd, max_pos=512, attn_scale=hd ** -0.5)
     prompt = list(np.random.default_rng(0).integers(0, m.cfg["vocab"], 300))
     dev = H.Dev(0)
     try:
@@ -207,3 +208,50 @@ def test_prefill_256_rows_engine():
     want, gaps = spec_loop.greedy(step, prompt, 4)
     assert min(gaps) > 4e-2
     assert got.tolist() == want
+
+
+def logits_of_prefixes(m, lengths, max_positions):
+    """forward_logits of the first n of max(lengths) tokens, for each n on one
+    engine in turn, against one oracle pass over all of them (row n - 1 sees
+    the n tokens before it)."""
+    from gpu_util import device_model
+    tokens = np.random.default_rng(5).integers(0, m.cfg["vocab"], max(lengths)).astype(np.int32)
+    pages = -(-max(lengths) // 16)
+    kv = O.HostKV(m, n_pages=pages, batch=1, max_pages_per_seq=pages)
+    kv.page_table[0] = np.arange(pages)
+    O.set_threads(16)
+    try:
+        want = O.verify_forward(m, kv, tokens[None], np.array([0], np.int32))[0]
+    finally:
+        O.set_threads(1)
+    dev = H.Dev(0)
+    try:
+        dm = device_model(dev, m)
+        eng = E.Engine(dev, dm.desc, None, max_positions=max_positions, draft_tokens=K)
+        for n in lengths:
+            got, top = eng.forward_logits(tokens[:n], m.cfg["vocab"])
+            err = np.abs(got - want[n - 1]).max()
+            say("prompt of", n, "max_abs logits", err)
+            assert err <= 2e-2 and top == np.argmax(got)
+        eng.close()
+    finally:
+        dev.close()
+
+
+@pytest.mark.parametrize("wfmt,afmt", [(O.W_I8PC, O.A_F16), (O.W_I4G128, O.A_F16)], ids=["i8", "i4"])
+def test_prefill_several_prompt_steps(wfmt, afmt):
+    """Prompts past the 2,048 tokens of a step: the steps before the last leave it
+    17 tokens at least (2,049 = 2,032 + 17; 4,097 = 2,048 + 2,032 + 17), which see
+    the whole cache, and shorter ones on the same engine after longer ones."""
+    from test_gpu_verify import small_model
+    m = small_model(wfmt, afmt, max_pos=4112, attn_scale=0.125)
+    logits_of_prefixes(m, [4097, 2048, 2049, 2064, 2065, 16, 17], 4112)
+
+
+def test_prefill_256_rows_lengths():
+    """The 256-row path (head_dim 96) at lengths on either side of its parts: no
+    whole part, one, two (the fewest it takes), 16, a second launch, and a longer
+    prompt after shorter ones (the parts' copies of the page-table row lag it)."""
+    from test_gpu_verify import small_model
+    m = small_model(O.W_I8PC, O.A_F16, hd=96, max_pos=640, attn_scale=96 ** -0.5)
+    logits_of_prefixes(m, [16, 32, 33, 40, 257, 258, 289, 300, 600, 33], 640)

@@ -88,9 +88,9 @@ def test_loaded_model_verify_step(dev, tmp_path, fmt, tied):
     lm.lm.close()
 
 
-def test_head_dim_96_through_the_vector_attention(dev, tmp_path):
+def test_head_dim_96_from_directory(dev, tmp_path):
     """A head size the reference refuses (96): loaded, and verified against
-    the oracle through the attention's vector path."""
+    the oracle."""
     m = small_model(O.W_I8PC, O.A_F16, hidden=384, heads=(4, 2), hd=96, attn_scale=96 ** -0.5)
     d = W.write_model_dir(str(tmp_path / "m"), m)
     lm = Loaded(dev, d)
