@@ -20,8 +20,9 @@
  *     are invalid): a token id outside the vocabulary (OPURE_E_INVALID; its
  *     row reads NaN), a row position seq_len + j at or past max_ctx or with no
  *     page in the page table (OPURE_E_CAPACITY; its K/V are not written and
- *     its attention is clamped), a bounded wait between waves that gave up
- *     (OPURE_E_DEVICE).
+ *     its attention is clamped), a bounded wait between waves or workgroups
+ *     that gave up (OPURE_E_DEVICE; the GEMVs, rejection, sampling, and greedy
+ *     acceptance inside the LM head or over stored logits).
  *     Uploads and downloads are synchronous, like UploadToBuffer /
  *     ReadbackFromBuffer (Opure_Dx12.h:230-244).
  *
@@ -439,9 +440,10 @@ int opure_profile_read(opure_dev* dev, uint32_t counts[OPURE_STAGE_COUNT], doubl
 int opure_debug_workspace(opure_dev* dev, void** ptr, uint64_t* bytes);
 /* Sleeps a bounded wait takes before it gives up (default 4M): between the
  * waves of a GEMV workgroup, between the slices of a sequence in the
- * one-launch rejection step, or in the LM head's greedy acceptance.  A test hook: 0 makes any wait that is not already met give
- * up at once, so the failure report can be checked while every wave still
- * runs to its end. */
+ * one-launch rejection step or of a row in opure_sample_rows, or in a greedy
+ * acceptance (the LM head's, or over stored logits).  A test hook: 0 makes any
+ * wait that is not already met give up at once, so the failure report can be
+ * checked while every wave still runs to its end. */
 int opure_debug_set_wait_limit(opure_dev* dev, uint32_t sleeps);
 /* GEMV engine of opure_gemv_batched_* at M <= 8 rows with a STORE / RESIDUAL /
  * SWIGLU epilogue: the matrix-core kernels (default) or the vector-ALU kernel

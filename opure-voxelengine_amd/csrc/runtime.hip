@@ -86,11 +86,11 @@ int check_device_errors(opure_dev* dev)
         hipError_t e = reset_acc_sync(dev);
         if (e == hipSuccess && dev->rej_sync) e = hipMemsetAsync(dev->rej_sync, 0, REJ_SYNC_BYTES, dev->stream);
         if (e == hipSuccess) e = hipStreamSynchronize(dev->stream);
-        if (e != hipSuccess) return hip_fail(e, "resetting the in-launch acceptance state");
+        if (e != hipSuccess) return hip_fail(e, "resetting the state that launches exchange");
     }
     if (w[ERR_WAIT])
-        return set_error(OPURE_E_DEVICE, "a bounded wait gave up (between a GEMV's waves, between a rejection "
-                         "step's slices, or in the LM head's greedy acceptance; after %u sleeps): that launch's "
+        return set_error(OPURE_E_DEVICE, "a bounded wait gave up (between a GEMV's waves, between the slices of a "
+                         "rejection step or of sampling, or in a greedy acceptance; after %u sleeps): that launch's "
                          "outputs are invalid%s%s", dev->wait_limit,
                          w[ERR_TOKEN] ? "; a token id was outside the vocabulary" : "",
                          w[ERR_POSITION] ? "; a position reached past max_ctx or the page table" : "");

@@ -149,6 +149,58 @@ def test_rejection_wait_gives_up_then_recovers(dev):
         buf.free()
 
 
+@pytest.mark.parametrize("kind", ["sample", "greedy", "greedy-in-step"])
+def test_sliced_wait_gives_up_then_recovers(dev, kind):
+    """Sampling and greedy acceptance over logits: slices of a row wait for each
+    other with the same bounded wait and share their words.  At 0 sleeps the
+    launch completes and the sync reports it, naming what waits (unless every
+    wait happened to be met); the state starts afresh, so the same call and the
+    other kind at the default limit equal the oracle bit for bit."""
+    rng = np.random.default_rng(4)
+    L = H.lib()
+    B, K, V = 24, 4, 128256
+    lg = (rng.standard_normal((B, K + 1, V)) * 3).astype(np.float32)
+    lb = dev.upload(lg)
+    drafts = lg[:, :K].argmax(2).astype(np.int32)
+    drafts[::2, 2] += 1
+    db, ot, ac = dev.upload(drafts), dev.alloc(B * (K + 1) * 4), dev.alloc(B * 4)
+    pos, seq = rng.integers(0, 999, B).astype(np.uint32), np.arange(B, dtype=np.uint32)
+    pb, sb, so = dev.upload(pos), dev.upload(seq), dev.alloc(B * 4)
+    ga = H.AcceptArgs(B, K, V, int(lb), None, int(db), K, 1.0, 0, None, int(ot), int(ac), None)
+    sa = H.SampleArgs(B, V, int(lb), 0.8, 3, int(pb), int(sb), 0, int(so))
+    w_out, w_acc = O.accept_greedy(lg, drafts)
+    w_ids = O.sample_rows(lg.reshape(-1, V)[:B], 0.8, 3, pos, seq, 0)
+    m, kv, dkv, run = small_step(dev, B=4, R=6, max_ctx=256)
+    tokens, lens = rng.integers(0, m.cfg["vocab"], (4, 6)), [100, 7, 200, 31]
+    step = lambda: launch(dev, run, tokens, lens, accept=H.ACCEPT_GREEDY)
+    greedy = lambda: H.check(L.opure_accept_greedy(dev.h, C.byref(ga)))
+    sample = lambda: H.check(L.opure_sample_rows(dev.h, C.byref(sa)))
+    H.check(L.opure_debug_set_wait_limit(dev.h, 0))
+    try:
+        {"sample": sample, "greedy": greedy, "greedy-in-step": step}[kind]()
+        code = sync_code(dev)
+        assert code in (H.OK, H.E_DEVICE)
+        if code == H.E_DEVICE:
+            msg = L.opure_last_error()
+            assert b"gave up" in msg and b"sampling" in msg and b"greedy acceptance" in msg
+    finally:
+        H.check(L.opure_debug_set_wait_limit(dev.h, 1 << 22))
+    for _ in range(2):
+        sample()
+        greedy()
+        assert sync_code(dev) == H.OK
+        assert np.array_equal(dev.download(so, np.int32, (B,)), w_ids)
+        assert np.array_equal(dev.download(ac, np.int32, (B,)), w_acc)
+        assert np.array_equal(dev.download(ot, np.int32, (B, K + 1)), w_out)
+        step()
+        assert sync_code(dev) == H.OK
+        out, acc = run.get_accept()
+        s_out, s_acc = O.accept_greedy(run.get_logits(), np.ascontiguousarray(tokens[:, 1:], np.int32))
+        assert np.array_equal(out, s_out) and np.array_equal(acc, s_acc)
+    for buf in (lb, db, ot, ac, pb, sb, so):
+        buf.free()
+
+
 def test_graph_survives_workspace_growth(dev):
     """A step captured into a graph, then an eager call that needs a larger
     workspace: the graph still replays to the eager result of its own shape."""
