@@ -371,8 +371,12 @@ int opure_verify_step(opure_dev* dev, const opure_verify_args* a);
  *      at positions seq_len[0] .. seq_len[0] + rows - 1 through the layers,
  *      their K/V appended; with `logits`, the last row's logits and (out_token)
  *      their argmax.  A prefill: the verify step with logits == NULL does the
- *      same for up to OPURE_MAX_BATCH_ROWS rows.  Quantised weights, 16-bit activations, head_dim 64 or 128,
- *      OPURE_MAX_ROWS + 1 .. OPURE_MAX_PROMPT_ROWS rows. */
+ *      same for up to OPURE_MAX_BATCH_ROWS rows.  Quantised weights, 16-bit
+ *      activations, head_dim 64 or 128, OPURE_MAX_ROWS + 1 ..
+ *      OPURE_MAX_PROMPT_ROWS rows.  The sums' order follows `rows` and max_ctx:
+ *      the same call gives the same bits, but a token's K/V may differ in their
+ *      last bits from those of a step over more or fewer rows, or of a verify
+ *      step. */
 #define OPURE_MAX_PROMPT_ROWS 2048
 typedef struct opure_prompt_args {
     const opure_model* model;

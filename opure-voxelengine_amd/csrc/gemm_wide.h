@@ -13,14 +13,15 @@
 //  set of 4 waves covers the row group (more than 64 rows of X): wave w multiplies
 //  tiles 2w, 2w + 1 by all of the group's column tiles, so it keeps 16 accumulator
 //  tiles, loads each weight byte once and reads each B fragment once per block for
-//  two MFMAs.  Fewer rows take one weight tile a wave, a prompt's
-//  rows four on a 2 x 2 wave grid (WideShape).  Weights go straight from HBM into
-//  registers: every wave loads its own tiles' 16 bytes a lane per block, in static register slots DW
-//  blocks ahead.  X goes through LDS: per block the set loads its column
-//  group's fragments into registers DX blocks ahead and writes them into a
-//  two-stage ring laid out fragment by fragment, 16 bytes a lane.  One barrier
-//  per block separates a stage's writes from its reads and the reads of two
-//  blocks back from the next writes.  The int8 kernel runs two such sets on
+//  two MFMAs.  Fewer rows take one weight tile a wave, an int8 prompt's of more
+//  than 256 rows four on a 2 x 2 wave grid (WideShape).  Weights go straight from
+//  HBM into registers: every wave loads its own tiles' 16 bytes a lane per block,
+//  in static register slots DW steps ahead.  X goes through LDS: per block the
+//  set loads its column group's fragments into registers DX steps ahead and
+//  writes them into a two-stage ring laid out fragment by fragment, 16 bytes a
+//  lane.  One barrier per step (one block, or two at one weight tile a wave)
+//  separates a stage's writes from its reads and the reads of two steps back
+//  from the next writes.  Up to 256 rows the int8 kernel runs two such sets on
 //  alternate K blocks (KH = 2, two waves a SIMD) and adds them at the end.
 //
 //  The budget per block of a workgroup is L2 -> CU traffic (8 KB of weights
@@ -31,11 +32,13 @@
 //  With one split the epilogue runs here; with several, each split writes
 //  its raw accumulators and k_wide_reduce adds the splits in split order and
 //  runs the epilogue (k_wide_reduce_norm for a residual that feeds an
-//  rmsnorm: it also writes the normalised rows).  The split count depends on
-//  the weight shape only, and each (row, column) sums its blocks in a fixed
-//  order (each wave set's blocks in order, then the sets added), so a row's
-//  result does not depend on how many rows share the call, and runs are
-//  reproducible.
+//  rmsnorm: it also writes the normalised rows).  Each (row, column) sums its
+//  blocks in a fixed order, so runs are reproducible.  For 17 to 256 rows the
+//  split count depends on the weight shape only and every kernel shape has the
+//  same order (each wave set's blocks in order, then the sets added), so a row's
+//  result does not depend on how many rows share the call.  A prompt's step of
+//  more rows takes its splits from the row count and, in int8, adds all blocks of
+//  a split in one chain: a row's last bits then depend on the step's rows.
 // ============================================================================
 #pragma once
 
@@ -88,7 +91,7 @@ struct WParams {
     uint32_t bps;     // blocks per split
     uint32_t part_rows;  // splits > 1: 0 = accumulators [split][tile][mt][64] lanes, 1 = [split][M][out] rows
     f4_t* part;       // splits > 1: the splits' accumulators
-    uint32_t prompt;  // host: more rows than a batch (a prompt's step)
+    uint32_t prompt;  // host: more than OPURE_MAX_BATCH_ROWS rows (a prompt's step)
 };
 
 // Workgroup -> (split, row group, column group).  Workgroups are dispatched
@@ -432,8 +435,9 @@ __global__ __launch_bounds__(256) void k_wide_reduce(WParams wp)
 // (g0 + g1) + (g2 + g3) -- then inv_rms from the tile sums in inv_rms_wave's
 // order and round(y * inv * gain) as k_rmsnorm_rows, so y, ss_out and the
 // normalised rows equal the separate passes' bit for bit.
-// RN_THREADS 1024 for batches of fewer rows than CUs, 256 past that: a few rows
-// are one round trip of each thread's loads, so fewer a thread.
+// RN_THREADS 1024 up to 128 rows, 256 past that: a few rows are one round trip
+// of each thread's loads, so fewer a thread (8B layer, fp16, at 20 rows 95.5 ->
+// 94.1 us, at 128 228.1 -> 226.9; at 160 and 256 rows within 1% either way).
 constexpr uint32_t RN_SPLITS = 8;   // the plan splits K at most 8 ways
 template <int WF, int AF, int UNITS, uint32_t RN_THREADS>
 __global__ __launch_bounds__(RN_THREADS) void k_wide_reduce_norm(WParams wp, const float* gain, void* xn)
@@ -530,8 +534,7 @@ int launch_wide_reduce_norm(opure_dev* dev, const WParams& wp, const float* gain
 template <int WF, int AF, int EPI>
 int launch_wide_epi_only(opure_dev* dev, const WParams& wp)
 {
-    // the kernel shape by the column tiles a workgroup has; every shape sums a
-    // row's blocks in the same order
+    // the kernel shape by the column tiles a workgroup has
     auto go = [&](auto sh) {
         using SH = decltype(sh);
         WParams q = wp;
@@ -549,6 +552,8 @@ int launch_wide_epi_only(opure_dev* dev, const WParams& wp)
         if (wp.prompt && wp.cgs <= 4u) return go(WideShape<4, 2, 2, 1>{});
         if (wp.prompt) return go(WideShape<4, 4, 2, 1>{});
     }
+    // the shapes of 17 to 256 rows (and a longer uint4 prompt's): one order of
+    // a row's blocks
     if (wp.cgs <= 2u) return go(WideShape<1, 2, 1, KH>{});
     if (wp.cgs <= 4u) return go(WideShape<1, 4, 1, KH>{});
     return go(WideShape<2, 8, 1, KH>{});

@@ -239,8 +239,9 @@ Plan make_plan(const opure_dev* dev, uint32_t wfmt, uint32_t xfmt, uint32_t out,
 
 // Shape plan of the GEMV over more than OPURE_MAX_ROWS rows: row groups of 8
 // tiles, column groups of at most 8 column tiles, and K splits for shapes
-// with few row groups.  The splits depend on the weight shape only (not on
-// the row count), so a row's sums do not depend on the batch around it.
+// with few row groups.  Up to OPURE_MAX_BATCH_ROWS rows the splits depend on the
+// weight shape only (not on the row count), so a row's sums do not depend on
+// the batch around it; past that (a prompt's step) they follow the row count.
 struct WidePlan {
     uint32_t tiles = 0, nblk = 0, mt = 0, nrg = 0, ncg = 0, cgs = 0, splits = 1, bps = 0;
     uint64_t part_bytes = 0;

@@ -125,7 +125,8 @@ __global__ __launch_bounds__(256) void k_tile_sumsq(const float* x, uint32_t M, 
 // k_tile_sumsq and the rmsnorm rows pass (gemv.hip) in one: a workgroup a row,
 // a thread a 16-column tile (h <= 4096), the tile sums in inv_rms_wave's order,
 // round(x * inv * gain) -- the bits of the two launches.  For the layer that
-// starts from a caller's residual over more than OPURE_MAX_ROWS rows.
+// starts from a caller's residual over more than OPURE_MAX_ROWS rows: a launch
+// less (8B layer at 20 rows 97.1 -> 94.1 us, at 256 324 -> 320; 1B 60.7 -> 57.7).
 template <int AF>
 __global__ __launch_bounds__(256) void k_norm_rows(const float* x, const float* gain, uint32_t h, float eps, void* xn)
 {
