@@ -123,7 +123,7 @@ __global__ __launch_bounds__(SH::NTH) __attribute__((amdgpu_waves_per_eu(2))) vo
     constexpr uint32_t SB = WD::SB, DW = WD::DW, DX = WD::DX, U = WD::U, KH = SH::KH;
     static_assert(U % 2 == 0 && U % DX == 0 && U % DW == 0, "static slots and stages");
     constexpr bool GS = WF == OPURE_W_I4G128;      // group sums of X
-    static_assert(XR >= 1 && TB % 2 == 0, "whole chunks a thread; the halves exchange half of the column tiles");
+    static_assert(XR >= 1 && TB % 2 == 0, "whole chunks a thread; the halves exchange half of the tiles");
     static_assert(KH == 1 || 4u * TA * TB * 64u <= KH * 2u * STAGE, "the halves' exchange reuses the X stages");
     static_assert(!GS || CH == 16u, "a DPP row of lanes stages one X row's group");
     __shared__ u4_t xl[KH * 2 * SB * STAGE];
@@ -147,15 +147,22 @@ __global__ __launch_bounds__(SH::NTH) __attribute__((amdgpu_waves_per_eu(2))) vo
     // slot rr ^ c of its fragment: the 8 chunks of a row land in 8 bank groups, and a fragment
     // read (lane (g4, r16) takes chunk NMF g4 + q of row r16) still reads 16 distinct slots.
     // Rows past M (or past the group's column tiles) read row M - 1 again: their columns are
-    // computed and never stored.
+    // computed and never stored.  Two wave sets of two weight tiles (int8 past 64 rows) put
+    // zeros in their place: products of zeros run faster than the row's again (LM head 128,256
+    // x 2,048 at 65 rows 84.9 -> 81.6 us, gate/up 16,384 x 2,048 at 144 21.2 -> 20.9; with no
+    // row past M the selects cost up to 1%).  The other shapes lose more by the selects (int8
+    // gate/up at 48 rows 10.1 -> 10.8, uint4 down 4,096 x 14,336 at 128 54.1 -> 56.5).
+    constexpr bool XZ = KH == 2u && TA == 2u;
     uint64_t xrow[XR];
     uint32_t xdst[XR];
+    bool xzero[XR];
 #pragma unroll
     for (uint32_t u = 0; u < XR; ++u)
     {
         const uint32_t e = u * 256u + tid;
         const uint32_t c = e % CH, rr = (e / CH) & 15u, ctl = e / (16u * CH);
         const uint32_t m = 16u * (ct0 + ctl) + rr;
+        xzero[u] = XZ && (ctl >= cn || m >= p.M);
         xrow[u] = (static_cast<uint64_t>(min(m, p.M - 1u)) * p.in + 8u * c) * 2u;
         xdst[u] = (ctl * NMF + c % NMF) * 64u + (c / NMF) * 16u + (rr ^ (c & 15u));
     }
@@ -176,7 +183,7 @@ __global__ __launch_bounds__(SH::NTH) __attribute__((amdgpu_waves_per_eu(2))) vo
 #pragma unroll
         for (uint32_t u = 0; u < XR; ++u)
         {
-            xh[st * STAGE + xdst[u]] = v[u];
+            xh[st * STAGE + xdst[u]] = xzero[u] ? u4_t{0u, 0u, 0u, 0u} : v[u];
             if constexpr (GS)
             {
                 const float s = unit_sum<AF>(v[u][0], v[u][1], v[u][2], v[u][3]);
@@ -304,15 +311,22 @@ __global__ __launch_bounds__(SH::NTH) __attribute__((amdgpu_waves_per_eu(2))) vo
         }
     };
 
+    // the two halves share the epilogue by weight tiles where a wave has two, so
+    // that a column group of 5 tiles is shared evenly too (by column tiles, 4 and
+    // 1, int8 gate/up 16,384 x 2,048 at 80 rows takes 21.3 us instead of 20.1, at
+    // 144 22.4 instead of 20.9), else by column tiles
+    constexpr bool BYT = KH == 2u && TA % 2u == 0u;
+    constexpr uint32_t FT = BYT ? TA / 2u : TA, FB = KH == 2u && !BYT ? TB / 2u : TB;   // tiles a wave finishes
+    const uint32_t a0 = BYT ? kh * FT : 0u, j0 = KH == 2u && !BYT ? kh * FB : 0u;
     // int8 with one split: the row scales of the tiles this wave finishes, loaded
     // now rather than after the K loop (a round trip off the epilogue)
-    f4_t scl[TA];
+    f4_t scl[FT];
     if constexpr (WF == OPURE_W_I8PC)
     {
 #pragma unroll
-        for (uint32_t a = 0; a < TA; ++a)
+        for (uint32_t a = 0; a < FT; ++a)
         {
-            const uint32_t t = min(tile0 + a, p.tiles - 1u);
+            const uint32_t t = min(tile0 + a0 + a, p.tiles - 1u);
 #pragma unroll
             for (int i = 0; i < 4; ++i) scl[a][i] = f16_to_f32(static_cast<const uint16_t*>(p.sc)[t * 16u + 4u * g4 + i]);
         }
@@ -322,38 +336,50 @@ __global__ __launch_bounds__(SH::NTH) __attribute__((amdgpu_waves_per_eu(2))) vo
     // halves SB blocks on, with one barrier for the whole workgroup.
     const uint32_t steps = (b_end - b_begin + KH * SB - 1u) / (KH * SB);
     const uint32_t bh = b_begin + kh;
-    u4_t xr[DX][SB][XR];
-    u4_t wv[DW][SB][TA], sv[DW][SB][TA];
-    auto block = [&](uint32_t step, uint32_t k) { return bh + KH * (SB * step + k); };
+    u4_t xr[DX * SB][XR];
+    u4_t wv[DW * SB][TA], sv[DW * SB][TA];
+    // slot SB d + k: block k of the d-th step ahead, bh + KH (SB d + k)
 #pragma unroll
-    for (uint32_t d = 0; d < DX; ++d)
+    for (uint32_t d = 0; d < DX * SB; ++d) xload(xr[d], bh + KH * d);
 #pragma unroll
-        for (uint32_t k = 0; k < SB; ++k) xload(xr[d][k], block(d, k));
-#pragma unroll
-    for (uint32_t d = 0; d < DW; ++d)
-#pragma unroll
-        for (uint32_t k = 0; k < SB; ++k) wload(wv[d][k], sv[d][k], block(d, k));
+    for (uint32_t d = 0; d < DW * SB; ++d) wload(wv[d], sv[d], bh + KH * d);
     for (uint32_t i0 = 0; i0 < steps; i0 += U)
     {
 #pragma unroll
         for (uint32_t s = 0; s < U; ++s)
         {
-            const uint32_t st = (s & 1u) * SB;
+            const uint32_t b = bh + KH * SB * (i0 + s), st = (s & 1u) * SB, xs = s % DX * SB, ws = s % DW * SB;
+            if constexpr (SB == 1u && TA == 2u)
+            {
+                // the loops below over one block, written out: the compiler
+                // schedules it better (int8 gate/up 28,672 x 4,096 at 256 rows
+                // 69.5 -> 68.0 us; uint4 at 256 87.5 -> 86.2, LM head 317 -> 310;
+                // a prompt's shapes of four weight tiles lose up to 1% by it)
+                xstore(xr[xs], st);
+                xload(xr[xs], b + KH * DX);
+                __syncthreads();
+                if (b < b_end) compute(wv[ws], sv[ws], st);
+                wload(wv[ws], sv[ws], b + KH * DW);
+            }
+            else
+            {
 #pragma unroll
-            for (uint32_t k = 0; k < SB; ++k) xstore(xr[s % DX][k], st + k);
+                for (uint32_t k = 0; k < SB; ++k) xstore(xr[xs + k], st + k);
 #pragma unroll
-            for (uint32_t k = 0; k < SB; ++k) xload(xr[s % DX][k], block(i0 + s + DX, k));
-            __syncthreads();
+                for (uint32_t k = 0; k < SB; ++k) xload(xr[xs + k], b + KH * (SB * DX + k));
+                __syncthreads();
 #pragma unroll
-            for (uint32_t k = 0; k < SB; ++k)
-                if (block(i0 + s, k) < b_end) compute(wv[s % DW][k], sv[s % DW][k], st + k);
+                for (uint32_t k = 0; k < SB; ++k)
+                    if (b + KH * k < b_end) compute(wv[ws + k], sv[ws + k], st + k);
 #pragma unroll
-            for (uint32_t k = 0; k < SB; ++k) wload(wv[s % DW][k], sv[s % DW][k], block(i0 + s + DW, k));
+                for (uint32_t k = 0; k < SB; ++k) wload(wv[ws + k], sv[ws + k], b + KH * (SB * DW + k));
+            }
         }
     }
 
+    // a, j: the tile's index among the ones that this wave finishes
     auto finish = [&](uint32_t a, uint32_t j, const f4_t& tot) {
-        const uint32_t tile = tile0 + a, cl = TB * wc + j;
+        const uint32_t tile = tile0 + a0 + a, cl = TB * wc + j0 + j;
         if (tile >= p.tiles || cl >= cn) return;
         const uint32_t ct = ct0 + cl;
         if (wp.splits == 1u)
@@ -384,28 +410,27 @@ __global__ __launch_bounds__(SH::NTH) __attribute__((amdgpu_waves_per_eu(2))) vo
     else
     {
         // the halves add through LDS (the X stages are free): half 0 finishes
-        // the first TB/2 column tiles of its wave, half 1 the others; each sum
-        // is (even blocks) + (odd blocks)
-        constexpr uint32_t HB = TB / 2u;
+        // the first half of its wave's weight or column tiles, half 1 the others;
+        // each sum is (even blocks) + (odd blocks)
+        constexpr uint32_t UA = BYT ? FT : 0u, UB = BYT ? 0u : FB;   // from half 0's tiles to half 1's
         __syncthreads();
-        u4_t* ex = xl + ((1u - kh) * 4u + w4) * (TA * HB * 64u);  // the other half's inbox for this wave
+        u4_t* ex = xl + ((1u - kh) * 4u + w4) * (FT * FB * 64u);  // the other half's inbox for this wave
 #pragma unroll
-        for (uint32_t a = 0; a < TA; ++a)
+        for (uint32_t a = 0; a < FT; ++a)
 #pragma unroll
-            for (uint32_t j = 0; j < HB; ++j)
-                ex[(a * HB + j) * 64u + lane] = __builtin_bit_cast(u4_t, kh == 0 ? acc[a][HB + j] : acc[a][j]);
+            for (uint32_t j = 0; j < FB; ++j)
+                ex[(a * FB + j) * 64u + lane] = __builtin_bit_cast(u4_t, kh == 0 ? acc[UA + a][UB + j] : acc[a][j]);
         __syncthreads();
-        const u4_t* in = xl + (kh * 4u + w4) * (TA * HB * 64u);
-        const uint32_t keep = kh == 0 ? 0u : HB;
+        const u4_t* in = xl + (kh * 4u + w4) * (FT * FB * 64u);
 #pragma unroll
-        for (uint32_t a = 0; a < TA; ++a)
+        for (uint32_t a = 0; a < FT; ++a)
 #pragma unroll
-            for (uint32_t j = 0; j < HB; ++j)
+            for (uint32_t j = 0; j < FB; ++j)
             {
-                const f4_t other = __builtin_bit_cast(f4_t, in[(a * HB + j) * 64u + lane]);
-                const f4_t mine = kh == 0 ? acc[a][j] : acc[a][HB + j];
+                const f4_t other = __builtin_bit_cast(f4_t, in[(a * FB + j) * 64u + lane]);
+                const f4_t mine = kh == 0 ? acc[a][j] : acc[UA + a][UB + j];
                 const f4_t even = kh == 0 ? mine : other, odd = kh == 0 ? other : mine;
-                finish(a, keep + j, even + odd);
+                finish(a, j, even + odd);
             }
     }
 }
